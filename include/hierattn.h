@@ -306,15 +306,15 @@ int hier_qkv_prologue(const HierPrologueArgs* args, void* stream);
 /*   d_proj = r * dy - r^3 * a * sum(dy * a) / dim,                         */
 /* a = the projection plus the bf16 camera product, r = its inverse RMS.    */
 /* Writes d_proj (bf16 [S][H*D], the gradient of q(x) / k(x) and of the     */
-/* camera adapter's output) and per wave one fp32 row of gain-gradient      */
-/* partials ([hier_qk_prologue_bwd_waves][H*D], to be summed by the caller; */
-/* the camera-weight gradient is d_proj^T . cam, a plain GEMM).  Model dims */
-/* that are multiples of 512 up to 4096, head dim 64 or 128.                */
+/* camera adapter's output) and, per run of tokens_per_wave tokens, one fp32 */
+/* row of gain-gradient partials ([hier_qk_prologue_bwd_waves][H*D], to be   */
+/* summed by the caller; rows past the tokens are 0).  Model dims that are   */
+/* multiples of 512 up to 4096, head dim 64 or 128.                          */
 typedef struct HierPrologueBwdArgs {
   int32_t S, H, D;
   float eps;
   int32_t C;                       /* camera feature width (12) if cam          */
-  int32_t tokens_per_wave;         /* consecutive tokens per wave (>= 1)        */
+  int32_t tokens_per_wave;         /* consecutive tokens per partial row (>= 1) */
   const uint16_t* qx;              /* [S][H*D] bf16 forward inputs              */
   const uint16_t* kx;
   const uint16_t* cam;             /* [S][C] bf16 camera tokens or NULL         */
@@ -336,6 +336,23 @@ typedef struct HierPrologueBwdArgs {
 /* Rows of each dw_*_partial buffer for args (S, tokens_per_wave); -1 if invalid. */
 int hier_qk_prologue_bwd_waves(const HierPrologueBwdArgs* args);
 int hier_qk_prologue_bwd(const HierPrologueBwdArgs* args, void* stream);
+
+/* hier_qk_prologue_bwd, then the sums of its partial rows as bf16: the gain */
+/* gradients and, when dw_cam_q / dw_cam_k are given, the camera weights'    */
+/* gradients d_proj^T . cam (attention.py:307-320), summed in the same pass. */
+/* S = 0 writes nothing.                                                     */
+typedef struct HierPrologueGradArgs {
+  uint16_t* dnorm_q;               /* [H*D] bf16                                */
+  uint16_t* dnorm_k;
+  uint16_t* dw_cam_q;              /* [H*D][12] bf16, or both NULL              */
+  uint16_t* dw_cam_k;
+  float* dwc_q_partial;            /* [waves][12][H*D] fp32 workspace, 16-byte aligned */
+  float* dwc_k_partial;
+  int32_t* segments;               /* [2][waves][16] workspace                  */
+} HierPrologueGradArgs;
+
+int hier_qk_prologue_grads(const HierPrologueBwdArgs* args, const HierPrologueGradArgs* grads,
+                           void* stream);
 
 /* ------------------------------------------------------------------------ */
 /* Block-sparse frame-causal flash attention forward over the tile list.    */

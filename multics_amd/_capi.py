@@ -143,6 +143,11 @@ class HierPrologueBwdArgs(C.Structure):
                [(n, vp) for n in ("dqx", "dkx", "dw_q_partial", "dw_k_partial")]
 
 
+class HierPrologueGradArgs(C.Structure):
+    _fields_ = [(n, vp) for n in ("dnorm_q", "dnorm_k", "dw_cam_q", "dw_cam_k", "dwc_q_partial",
+                                  "dwc_k_partial", "segments")]
+
+
 class HierMergeArgs(C.Structure):
     _fields_ = [(n, i32) for n in ("n_groups", "n_src", "rows", "rows_per_item")] + \
                [(n, vp) for n in ("items", "kv_idx", "kv_mask", "blk_and", "acc", "src_item",
@@ -168,6 +173,7 @@ EXPORTS = {
     "hier_qkv_prologue": [C.POINTER(HierPrologueArgs), vp],
     "hier_qk_prologue_bwd_waves": [C.POINTER(HierPrologueBwdArgs)],
     "hier_qk_prologue_bwd": [C.POINTER(HierPrologueBwdArgs), vp],
+    "hier_qk_prologue_grads": [C.POINTER(HierPrologueBwdArgs), C.POINTER(HierPrologueGradArgs), vp],
     "hier_attn_fwd": [C.POINTER(HierFwdArgs), vp],
     "hier_attn_bwd": [C.POINTER(HierBwdArgs), vp],
     "hier_attn_bwd_noalloc": [C.POINTER(HierBwdArgs), vp],

@@ -551,15 +551,23 @@ def gated_residual(x: torch.Tensor, gate: torch.Tensor, residual: torch.Tensor, 
     return out
 
 
-PROLOGUE_BWD_TOKENS_PER_WAVE = 16
+def _prologue_bwd_tokens(S: int, dim: int) -> int:
+    """Tokens of one workgroup of the prologue backward: its workgroups of
+    both projections fill the 256 CUs once with about six waves each (one
+    workgroup of 3072 channels, six of 512) -- HBM-bound already there, and
+    every workgroup writes fp32 rows of sums (18,816 x 3072: 159 us with 128
+    workgroups per projection, 170 with 256, 191 with 512, 209 with 64) -- of
+    at least 8 tokens."""
+    rows = 128 * max(1, 6 * 512 // dim)
+    return max(8, -(-S // rows))
 
 
 class QKPrologueFunction(torch.autograd.Function):
     """Differentiable q / k projection tail on the HIP kernels: forward
     ``hier_qkv_prologue`` (camera adapter, RMSNorm, gain, RoPE fused), backward
-    ``hier_qk_prologue_bwd`` (the same chain's gradient recomputed in fp32 from
-    the forward's inputs), plus the camera-weight gradient as the GEMM
-    ``d_proj^T . cam`` and the gains' column sums.  Replaces the autograd of
+    ``hier_qk_prologue_grads`` (the same chain's gradient recomputed in fp32
+    from the forward's inputs, with the gains' and the camera weights' sums
+    taken in the same pass).  Replaces the autograd of
     attention.py:355-365 / 307-320 / 231-242 and rope.py:248-254 on the
     training path.  Inputs: ``qx, kx`` [S, H*D] bf16 (the q / k projections),
     the RMSNorm gains, fp32 cos / sin [S, D/2], optional camera rows [S, 12]
@@ -595,30 +603,47 @@ class QKPrologueFunction(torch.autograd.Function):
         dq, dk = grads
         dqx = torch.empty_like(qx)
         dkx = torch.empty_like(kx)
+        if cam is not None:      # read as bf16, as the forward reads them
+            wcq16, wck16 = (w.to(torch.bfloat16).contiguous() for w in (wcq, wck))
+        nwq, nwk = wq.contiguous(), wk.contiguous()
         args = _capi.HierPrologueBwdArgs(
             S=S, H=H, D=D, eps=float(ctx.eps), C=0 if cam is None else cam.shape[-1],
-            tokens_per_wave=PROLOGUE_BWD_TOKENS_PER_WAVE, qx=qx.data_ptr(), kx=kx.data_ptr(),
+            tokens_per_wave=_prologue_bwd_tokens(S, dim), qx=qx.data_ptr(), kx=kx.data_ptr(),
             cam=None if cam is None else cam.data_ptr(),
-            w_cam_q=None if cam is None else wcq.data_ptr(),
-            w_cam_k=None if cam is None else wck.data_ptr(),
-            norm_q_w=wq.data_ptr(), norm_k_w=wk.data_ptr(), rope_cos=cs.data_ptr(),
+            w_cam_q=None if cam is None else wcq16.data_ptr(),
+            w_cam_k=None if cam is None else wck16.data_ptr(),
+            norm_q_w=nwq.data_ptr(), norm_k_w=nwk.data_ptr(), rope_cos=cs.data_ptr(),
             rope_sin=sn.data_ptr(), dq=dq.data_ptr(), dk=dk.data_ptr(), dq_ss=dq.stride(0),
             dq_sh=dq.stride(1), dk_ss=dk.stride(0), dk_sh=dk.stride(1), dqx=dqx.data_ptr(),
             dkx=dkx.data_ptr())
-        waves = int(_capi.lib().hier_qk_prologue_bwd_waves(C.byref(args)))
-        if waves < 0:
+        rows = int(_capi.lib().hier_qk_prologue_bwd_waves(C.byref(args)))
+        if rows < 0:
             raise NotImplementedError("prologue backward: too many tokens")
-        part = torch.empty((2, max(waves, 1), dim), dtype=torch.float32, device=dev)
-        args.dw_q_partial, args.dw_k_partial = part[0].data_ptr(), part[1].data_ptr()
-        _capi.call("hier_qk_prologue_bwd", C.byref(args), _stream(dev))
-        dw = part[:, :waves].sum(dim=1) if waves else torch.zeros((2, dim), device=dev)
-        dwq, dwk = (x.to(wq.dtype) for x in dw)
+        cam_w = cam is not None and (ctx.needs_input_grad[5] or ctx.needs_input_grad[6])
+        # workspace: per workgroup its sums of the gain gradient (one row) and
+        # the slots of its camera sums (12 rows and their tokens); results in
+        # bf16, [2, dim] / [2, dim, 12]
+        part = torch.empty((2, rows, 13 if cam_w else 1, dim), dtype=torch.float32, device=dev)
+        dw = torch.empty((2, dim), dtype=torch.bfloat16, device=dev)
+        dwc = torch.empty((2, dim, 12), dtype=torch.bfloat16, device=dev) if cam_w else None
+        flat = part.view(2, -1)
+        args.dw_q_partial, args.dw_k_partial = flat[0].data_ptr(), flat[1].data_ptr()
+        grads = _capi.HierPrologueGradArgs(dnorm_q=dw[0].data_ptr(), dnorm_k=dw[1].data_ptr())
+        if cam_w:
+            grads.dw_cam_q, grads.dw_cam_k = dwc[0].data_ptr(), dwc[1].data_ptr()
+            off = rows * dim * 4
+            grads.dwc_q_partial = flat[0].data_ptr() + off
+            grads.dwc_k_partial = flat[1].data_ptr() + off
+            seg = torch.empty((2, rows, 16), dtype=torch.int32, device=dev)
+            grads.segments = seg.data_ptr()
+        _capi.call("hier_qk_prologue_grads", C.byref(args), C.byref(grads), _stream(dev))
+        dwq, dwk = dw[0].to(wq.dtype), dw[1].to(wk.dtype)
         dwcq = dwck = dcam = None
         if cam is not None:
             if ctx.needs_input_grad[5]:
-                dwcq = torch.mm(dqx.t(), cam.to(dqx.dtype)).to(wcq.dtype)
+                dwcq = dwc[0].to(wcq.dtype)
             if ctx.needs_input_grad[6]:
-                dwck = torch.mm(dkx.t(), cam.to(dkx.dtype)).to(wck.dtype)
+                dwck = dwc[1].to(wck.dtype)
             if ctx.needs_input_grad[4]:
                 dcam = (torch.mm(dqx, wcq.to(dqx.dtype)) + torch.mm(dkx, wck.to(dkx.dtype))).to(
                     cam.dtype)

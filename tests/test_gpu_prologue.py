@@ -213,3 +213,59 @@ def test_prologue_backward_matches_fp32_autograd(camera, shape):
     if camera:
         _grad_check("dcam_q", hwcq.grad, rwcq.grad)
         _grad_check("dcam_k", hwck.grad, rwck.grad)
+
+
+@pytest.mark.parametrize("S,H,D,run", [
+    (1, 4, 128, 1),          # one token, one workgroup, three of its four padded rows empty
+    (8, 8, 64, 3),           # exactly one workgroup of 8 tokens, a camera row change inside a trip
+    (13, 8, 128, 1),         # every token its own camera row; a last trip of one token
+    (1030, 12, 128, 37),     # workgroups of 8 tokens, camera runs that cross them
+    (1100, 24, 128, 220),    # 9 tokens per workgroup: a ragged last trip in each
+    (70, 28, 128, 5),        # 8 channels per thread, two tokens per trip, odd runs
+    (70, 64, 64, 70),        # the largest model dim
+])
+def test_prologue_backward_sums(S, H, D, run):
+    """The sums over tokens of the prologue backward (gain and camera-weight
+    gradients) and the projections' gradients, where the token split, the
+    trips and the camera runs (``run`` tokens of one row, every third run
+    zeros) can go wrong, against float64 autograd.  Bounds: results are bf16
+    (2^-9 of the value) of fp32 sums of terms with the forward's bf16 rounding
+    of a (2^-9 of each term): 1 % of the largest entry."""
+    need_gpu()
+    from multics_amd.kernels import qk_prologue_train
+    say("prologue backward sums", S, H, D, run)
+    dim = H * D
+    g = torch.Generator().manual_seed(S + H)
+    bf = lambda *s, std=1.0: (std * torch.randn(*s, generator=g)).to(torch.bfloat16)
+    qx, kx = bf(S, dim), bf(S, dim)
+    wq, wk = (1 + 0.1 * torch.randn(2, dim, generator=g)).to(torch.bfloat16)
+    wcq, wck = bf(dim, 12, std=0.05), bf(dim, 12, std=0.05)
+    rows = bf(-(-S // run), 12)
+    rows[2::3] = 0
+    cam = rows.repeat_interleave(run, 0)[:S].contiguous()
+    ang = 6.283 * torch.rand(S, D // 2, generator=g, dtype=torch.float64)
+    cos, sin = ang.cos(), ang.sin()
+    dq, dk = bf(S, H, D), bf(S, H, D)
+    leaf = lambda t: t.cuda().requires_grad_(True)
+    hip = [leaf(t) for t in (qx, kx, wq, wk, wcq, wck)]
+    q, k = qk_prologue_train(hip[0], hip[1], norm_q_w=hip[2], norm_k_w=hip[3],
+                             rope_cos=cos.float().cuda(), rope_sin=sin.float().cuda(), num_heads=H,
+                             eps=1e-6, cam=cam.cuda(), w_cam_q=hip[4], w_cam_k=hip[5])
+    got = torch.autograd.grad((q, k), hip, (dq.cuda(), dk.cuda()))
+    torch.cuda.synchronize()
+
+    ref = [t.double().requires_grad_(True) for t in (qx, kx, wq, wk, wcq, wck)]
+
+    def tail(x, w, wc):
+        a = x + cam.double() @ wc.t()
+        z = (a * torch.rsqrt(a.square().mean(-1, keepdim=True) + 1e-6) * w).view(S, H, D // 2, 2)
+        c, s = cos[:, None], sin[:, None]
+        return torch.stack([z[..., 0] * c - z[..., 1] * s, z[..., 0] * s + z[..., 1] * c],
+                           -1).flatten(2)
+
+    want = torch.autograd.grad((tail(ref[0], ref[2], ref[4]), tail(ref[1], ref[3], ref[5])), ref,
+                               (dq.double(), dk.double()))
+    for name, a, b in zip(("dqx", "dkx", "dnorm_q", "dnorm_k", "dcam_q", "dcam_k"), got, want):
+        err = (a.double().cpu() - b).abs().max().item()
+        say(f"  {name}: max-abs {err:.3e} of {b.abs().max().item():.3e}")
+        assert err <= 1e-2 * b.abs().max().item(), name
