@@ -1,100 +1,415 @@
 // Frame-window attention of the action branches' cached attention
 // (multics/models/blocks.py:256-375: mouse temporal self-attention and
-// keyboard cross-attention over a rolling cache).  The sequences are short
-// (a few queries per sequence and head against at most a few hundred cached
-// keys), so instead of the tile kernel's 32 x 32 MFMA blocks a wave serves
-// 64 / (D/8) (sequence, query) slots of one head: each query owns D/8 lanes,
-// each lane 8 channels.  The partial dot products are summed across the
-// query's lanes and the softmax runs online in fp32.  For the temporal
-// branch the kernel is bound by reading the cached window once.
+// keyboard cross-attention over a rolling cache).  Key j is visible to query i
+// when k_frame[j] / n_block <= q_frame[i] / n_block and, with a window,
+// q_frame[i] - k_frame[j] < local_attn.  Scores, softmax weights and sums are
+// fp32 (the weights multiply V as two bf16 parts where the matrix cores do it).
+//
+// Two kernels, by the queries and keys of a sequence:
+//
+// seq_kernel    few queries (the temporal branch: one sequence per spatial
+//               token, a block's 3 frames against a window of 24).  Bound by
+//               reading K and V once.  One wave owns a (sequence, head) and up
+//               to 8 of its queries: it loads the window's rows at once (D / 8
+//               lanes per row, up to 8 groups of rows: 8 KB each of K and V),
+//               scores them for every query from registers and adds the row
+//               groups' sums at the end.  2,200 sequences x 24 heads of 128,
+//               3 x 24 keys: 128-136 us, 5.2-5.5 TB/s (155 us, 4.5 TB/s, when
+//               each query read the rows for itself, four keys at a time).
+// tile_kernel   more (the keyboard branch: 660 video tokens against 96 keyboard
+//               tokens per player): 128 queries per workgroup on the matrix
+//               cores, 64-key tiles of K and V in LDS, the next tile's rows
+//               loaded during the current one.  Bound by the latency of its
+//               few steps.  10 x 24 heads, 660 x 96 keys: 34 us (329 us with
+//               one key at a time per query).
 #include "hier_common.h"
+#include "hier_launch.h"
+#include "hier_tile.h"
+
+#include <climits>
 
 namespace {
 
-typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
-typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+using namespace hier::tile;
+
 constexpr float kLog2e = 1.4426950408889634f;
+constexpr float kNoMax = -1e30f;       // running max of a row without a visible key
 
 __device__ __forceinline__ float lo(uint32_t w) { return __uint_as_float(w << 16); }
 __device__ __forceinline__ float hi(uint32_t w) { return __uint_as_float(w & 0xffff0000u); }
-__device__ __forceinline__ uint32_t f2bf(float f) {
-  return (uint32_t)__builtin_bit_cast(uint16_t, (__bf16)f);
+
+// The key frames that a query sees are an interval [first, first + span]: the
+// block rule bounds them above (n_block divides towards zero, as the host's
+// integer division of non-negative frames does), the window below.  It always
+// holds the query's own frame.
+struct Window {
+  int first;
+  uint32_t span;
+  __device__ __forceinline__ void init(int qf, int n_block, int local_attn) {
+    const int b = qf / n_block;
+    const int64_t last = (int64_t)b * n_block + (b >= 0 ? n_block - 1 : 0);
+    const int64_t f0 = local_attn < 0 ? (int64_t)INT_MIN : (int64_t)qf - local_attn + 1;
+    first = (int)max(f0, (int64_t)INT_MIN);
+    span = (uint32_t)(min(last, (int64_t)INT_MAX - 1) - first);   // INT_MAX marks no key
+  }
+  __device__ __forceinline__ bool sees(int kf) const { return (uint32_t)(kf - first) <= span; }
+};
+
+template <int CTRL>
+__device__ __forceinline__ float dpp(float v) {
+  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xF, 0xF, true));
+}
+__device__ __forceinline__ float fold32(float a, float b) {   // lanes 0-31: a over both halves; 32-63: b
+  const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+  return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+}
+__device__ __forceinline__ float fold16(float a, float b) {   // rows 0, 2: a's pairs of rows; 1, 3: b's
+  const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+  return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+}
+__device__ __forceinline__ float max16(float v) {
+  const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
+}
+
+// ---- up to 8 queries per sequence ------------------------------------------
+
+// One wave: NQ queries of a (sequence, head), the keys in one chunk of G row
+// groups or (LOOP) in several.  A sequence's ceil(Lq / NQ) waves sit side by side (in one
+// workgroup as a rule), so its rows come from memory once.
+template <int D, int NQ, int G, bool LOOP>
+__global__ __launch_bounds__(256, LOOP || NQ > 4 ? 2 : 3) void seq_kernel(HierFrameAttnArgs a,
+                                                                     uint32_t nqg, uint32_t units) {
+  constexpr int LPR = D / 8;          // lanes per row
+  constexpr int R = 64 / LPR;         // rows per group
+  const int lane = threadIdx.x & 63;
+  const uint32_t unit = blockIdx.x * 4 + __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  if (unit >= units) return;
+  const uint32_t bh = unit / nqg, b = bh / (uint32_t)a.H;
+  const int h = (int)(bh - b * (uint32_t)a.H), q0 = (int)(unit - bh * nqg) * NQ;
+  const int c = lane % LPR, r = lane / LPR;
+  // rows stepped by a uniform stride; a lane past the last key repeats it, unseen
+  const uint16_t* const kb = a.k + (int64_t)b * a.k_sb + (int64_t)h * a.k_sh + 8 * c;
+  const uint16_t* const vb = a.v + (int64_t)b * a.v_sb + (int64_t)h * a.v_sh + 8 * c;
+  const uint16_t* const kl = kb + (int64_t)(a.Lk - 1) * a.k_ss;
+  const uint16_t* const vl = vb + (int64_t)(a.Lk - 1) * a.v_ss;
+  const uint16_t* const kr = kb + (int64_t)r * a.k_ss;
+  const uint16_t* const vr = vb + (int64_t)r * a.v_ss;
+  u32x4 k[G], v[G];
+  int kf[G];
+  auto fetch = [&](int j0) {          // a chunk's rows, all before any is used
+#pragma unroll
+    for (int g = 0; g < G; ++g)
+      k[g] = *reinterpret_cast<const u32x4*>(
+          j0 + g * R + r < a.Lk ? kr + (int64_t)(j0 + g * R) * a.k_ss : kl);
+#pragma unroll
+    for (int g = 0; g < G; ++g) kf[g] = a.k_frame[min(j0 + g * R + r, a.Lk - 1)];
+#pragma unroll
+    for (int g = 0; g < G; ++g)
+      v[g] = *reinterpret_cast<const u32x4*>(
+          j0 + g * R + r < a.Lk ? vr + (int64_t)(j0 + g * R) * a.v_ss : vl);
+  };
+  u32x4 q[NQ];
+#pragma unroll
+  for (int i = 0; i < NQ; ++i)
+    q[i] = *reinterpret_cast<const u32x4*>(a.q + (int64_t)b * a.q_sb +
+                                           (int64_t)min(q0 + i, a.Lq - 1) * a.q_ss +
+                                           (int64_t)h * a.q_sh + 8 * c);
+  const int qf = a.q_frame[min(q0 + min(lane, NQ - 1), a.Lq - 1)];   // lane i: query i
+  // a window of one chunk: its rows in flight before the first wait (as a
+  // loop's carried state they would cost as many registers again; the barrier
+  // keeps the compiler from moving V's loads to where they are used)
+  if (!LOOP && a.Lk > 0) fetch(0);
+  __builtin_amdgcn_sched_barrier(0);
+  Window win[NQ];
+  {
+    Window w;
+    w.init(qf, a.n_block, a.local_attn);
+#pragma unroll
+    for (int i = 0; i < NQ; ++i) {
+      win[i].first = __builtin_amdgcn_readlane(w.first, i);
+      win[i].span = (uint32_t)__builtin_amdgcn_readlane((int)w.span, i);
+    }
+  }
+  const float c2 = a.scale * kLog2e;
+  float m[NQ], l[NQ], o[NQ][8];
+#pragma unroll
+  for (int i = 0; i < NQ; ++i) {
+    m[i] = kNoMax;
+    l[i] = 0.f;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) o[i][e] = 0.f;
+  }
+  auto chunk = [&](int j0) {
+#pragma unroll
+    for (int g = 0; g < G; ++g) kf[g] = j0 + g * R + r < a.Lk ? kf[g] : INT_MAX;
+    float s[G][NQ], mx[NQ];
+#pragma unroll
+    for (int i = 0; i < NQ; ++i) mx[i] = -INFINITY;
+#pragma unroll
+    for (int g = 0; g < G; ++g) {
+#pragma unroll
+      for (int i = 0; i < NQ; ++i) {
+        float t = 0.f;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const uint32_t x = q[i][e], y = k[g][e];
+          t = __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2, x),
+                                              __builtin_bit_cast(bf16x2, y), t, false);
+        }
+        t += dpp<0xB1>(t);                      // the row's lanes: quad_perm [1,0,3,2]
+        t += dpp<0x4E>(t);                      // quad_perm [2,3,0,1]
+        if constexpr (LPR == 16) {
+          t += dpp<0x124>(t);                   // row_ror:4
+          t += dpp<0x128>(t);                   // row_ror:8
+        } else {
+          t += dpp<0x141>(t);                   // row_half_mirror
+        }
+        s[g][i] = win[i].sees(kf[g]) ? t * c2 : -INFINITY;
+        mx[i] = fmaxf(mx[i], s[g][i]);
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < NQ; ++i) {
+      if constexpr (LPR == 8) mx[i] = fmaxf(mx[i], dpp<0x128>(mx[i]));
+      const float mn = fmaxf(m[i], pair_max(max16(mx[i])));
+      const float alpha = __builtin_amdgcn_exp2f(m[i] - mn);
+      m[i] = mn;
+      l[i] *= alpha;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) o[i][e] *= alpha;
+    }
+#pragma unroll
+    for (int g = 0; g < G; ++g) {
+      float x[8];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const uint32_t w = v[g][e];
+        x[2 * e] = lo(w);
+        x[2 * e + 1] = hi(w);
+      }
+#pragma unroll
+      for (int i = 0; i < NQ; ++i) {
+        const float p = __builtin_amdgcn_exp2f(s[g][i] - m[i]);
+        l[i] += p;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) o[i][e] = fmaf(p, x[e], o[i][e]);
+      }
+    }
+  };
+  if constexpr (LOOP) {
+    for (int j0 = 0; j0 < a.Lk; j0 += G * R) {
+      fetch(j0);
+      chunk(j0);
+    }
+  } else if (a.Lk > 0) {
+    chunk(0);
+  }
+  // Sums over the row groups, four queries at a time: lane row 0 / 1 / 2 / 3
+  // (16 lanes) ends up with query 0 / 2 / 1 / 3 of the four, and stores it.
+  const int rw = lane >> 4, qr = (rw & 1) << 1 | rw >> 1;
+#pragma unroll
+  for (int i0 = 0; i0 < NQ; i0 += 4) {
+    auto fold = [&](auto get) {
+      float x[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        x[i] = i0 + i < NQ ? get(min(i0 + i, NQ - 1)) : 0.f;
+        if constexpr (LPR == 8) x[i] += dpp<0x128>(x[i]);
+      }
+      return fold16(fold32(x[0], x[1]), fold32(x[2], x[3]));
+    };
+    const float lt = fold([&](int i) { return l[i]; });
+    const float inv = lt > 0.f ? 1.f / lt : 0.f;
+    u32x4 w;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const float x = fold([&](int i) { return o[i][2 * e]; }) * inv;
+      const float y = fold([&](int i) { return o[i][2 * e + 1]; }) * inv;
+      w[e] = (uint32_t)f2bf(x) | ((uint32_t)f2bf(y) << 16);
+    }
+    if (i0 + qr < NQ && q0 + i0 + qr < a.Lq && (LPR == 16 || (lane & 8) == 0))
+      *reinterpret_cast<u32x4*>(a.o + (int64_t)b * a.o_sb + (int64_t)(q0 + i0 + qr) * a.o_ss +
+                                (int64_t)h * a.o_sh + 8 * c) = w;
+  }
+}
+
+// ---- more queries: matrix-core tiles ----------------------------------------
+//
+// Four waves of 32 queries.  S^T = K Q^T leaves each lane one query and 16 keys
+// of a 32-key block (hier_tile.h); P goes from the accumulators into the
+// operand of O^T += V^T P^T as the bf16 of P and the bf16 of what that rounding
+// left (2^-17 of P together: the products with bf16 V are exact, the sums
+// fp32).  The rows reach LDS through registers: any row stride works.
+
+template <int D>
+__global__ __launch_bounds__(256, 2) void tile_kernel(HierFrameAttnArgs a, int q_tiles, int total) {
+  constexpr int NC = Geo<D>::NC, NDB = Geo<D>::NDB, CPR = Geo<D>::CPR, ROWB = Geo<D>::ROWB;
+  constexpr int NL = kSlab * CPR / 256;     // 16-byte chunks per thread and tile
+  __shared__ __align__(16) char lds_k[Geo<D>::TILEB], lds_v[Geo<D>::TILEB];
+  __shared__ __align__(16) int lds_f[kSlab];
+  // the query tiles of one sequence and head on one XCD, which then reads
+  // their keys from memory once
+  const int logical = hier::xcd_logical(blockIdx.x, gridDim.x);
+  if (logical >= total) return;
+  const int bh = logical / q_tiles, b = bh / a.H, h = bh - b * a.H;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int q0 = (logical - bh * q_tiles) * 128 + wave * 32;
+  const bool active = q0 < a.Lq;
+  const int qi = min(q0 + (lane & 31), a.Lq - 1);
+  const uint16_t* const kb = a.k + (int64_t)b * a.k_sb + (int64_t)h * a.k_sh;
+  const uint16_t* const vb = a.v + (int64_t)b * a.v_sb + (int64_t)h * a.v_sh;
+  u32x4 kr[NL], vr[NL];
+  int fr = INT_MAX;
+  auto fetch = [&](int j0) {                // rows past the last repeat it, unseen
+#pragma unroll
+    for (int i = 0; i < NL; ++i) {
+      const int x = tid + 256 * i, row = min(j0 + x / CPR, a.Lk - 1), ch = x % CPR;
+      kr[i] = *reinterpret_cast<const u32x4*>(kb + (int64_t)row * a.k_ss + 8 * ch);
+      vr[i] = *reinterpret_cast<const u32x4*>(vb + (int64_t)row * a.v_ss + 8 * ch);
+    }
+    if (tid < kSlab) {
+      const int f = a.k_frame[min(j0 + tid, a.Lk - 1)];
+      fr = j0 + tid < a.Lk ? f : INT_MAX;
+    }
+  };
+  if (a.Lk > 0) fetch(0);
+  bf16x8 q[NC];
+  Window win;
+  {
+    const uint16_t* p = a.q + (int64_t)b * a.q_sb + (int64_t)qi * a.q_ss + (int64_t)h * a.q_sh +
+                        8 * (lane >> 5);
+#pragma unroll
+    for (int i = 0; i < NC; ++i) q[i] = *reinterpret_cast<const bf16x8*>(p + 16 * i);
+    win.init(a.q_frame[qi], a.n_block, a.local_attn);
+  }
+  const float c2 = a.scale * kLog2e;
+  int ka[NC], va[NDB];
+#pragma unroll
+  for (int i = 0; i < NC; ++i) ka[i] = row_read_off<D, kRowRead>(lane, i);
+#pragma unroll
+  for (int i = 0; i < NDB; ++i) va[i] = tr_read_off<D, kTrRead>(lane, i, 0);
+  constexpr int HALF = (8 / Geo<D>::NI) * ROWB;   // rows of keys +8
+  f32x16 o[NDB];
+#pragma unroll
+  for (int i = 0; i < NDB; ++i) o[i] = f32x16{};
+  float m = kNoMax, l = 0.f;
+  for (int j0 = 0; j0 < a.Lk; j0 += kSlab) {
+    __syncthreads();                        // every wave is done with the tile in LDS
+#pragma unroll
+    for (int i = 0; i < NL; ++i) {
+      const int x = tid + 256 * i, row = x / CPR, ch = x % CPR;
+      *reinterpret_cast<u32x4*>(lds_k + prow<D>(row) * ROWB + 16 * (ch ^ swz<D, kRowRead>(row))) = kr[i];
+      *reinterpret_cast<u32x4*>(lds_v + prow<D>(row) * ROWB + 16 * (ch ^ swz<D, kTrRead>(row))) = vr[i];
+    }
+    if (tid < kSlab) lds_f[tid] = fr;
+    __syncthreads();
+    if (j0 + kSlab < a.Lk) fetch(j0 + kSlab);
+    if (!active) continue;
+    // one 32-key block at a time (the last tile may hold one)
+#pragma unroll 1
+    for (int kb32 = 0; kb32 < 2 && j0 + 32 * kb32 < a.Lk; ++kb32) {
+      const char* kt = lds_k + kb32 * 32 * ROWB;
+      const char* vt0 = lds_v + kb32 * 32 * ROWB;
+      f32x16 s = {};
+#pragma unroll
+      for (int i = 0; i < NC; ++i) s = mfma(*reinterpret_cast<const bf16x8*>(kt + ka[i]), q[i], s);
+      float mx = -INFINITY;
+#pragma unroll
+      for (int g4 = 0; g4 < 4; ++g4) {
+        const u32x4 f = *reinterpret_cast<const u32x4*>(&lds_f[kb32 * 32 + 8 * g4 + 4 * (lane >> 5)]);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const float x = win.sees((int)f[e]) ? s[4 * g4 + e] * c2 : -INFINITY;
+          s[4 * g4 + e] = x;
+          mx = fmaxf(mx, x);
+        }
+      }
+      const float mn = fmaxf(m, pair_max(mx));
+      if (__ballot(mn > m) != 0) {
+        const float alpha = __builtin_amdgcn_exp2f(m - mn);
+        l *= alpha;
+#pragma unroll
+        for (int i = 0; i < NDB; ++i)
+#pragma unroll
+          for (int e = 0; e < 16; ++e) o[i][e] *= alpha;
+        m = mn;
+      }
+      bf16x8 ph[2], pl[2];
+#pragma unroll
+      for (int e = 0; e < 16; ++e) {
+        const float p = __builtin_amdgcn_exp2f(s[e] - m);
+        l += p;
+        const __bf16 t = (__bf16)p;
+        ph[e >> 3][e & 7] = t;
+        pl[e >> 3][e & 7] = (__bf16)(p - (float)t);
+      }
+#pragma unroll
+      for (int j = 0; j < 2; ++j)
+#pragma unroll
+        for (int i = 0; i < NDB; ++i) {
+          const char* p0 = vt0 + j * 16 * ROWB + va[i];
+          const bf16x8 vt = tr_read(p0, p0 + HALF);
+          o[i] = mfma(vt, ph[j], o[i]);
+          o[i] = mfma(vt, pl[j], o[i]);
+        }
+    }
+  }
+  if (q0 + (lane & 31) >= a.Lq) return;
+  const float lt = pair_sum(l);
+  const float inv = lt > 0.f ? 1.f / lt : 0.f;
+  uint16_t* op = a.o + (int64_t)b * a.o_sb + (int64_t)qi * a.o_ss + (int64_t)h * a.o_sh;
+#pragma unroll
+  for (int i = 0; i < NDB; ++i)
+#pragma unroll
+    for (int g4 = 0; g4 < 4; ++g4) {
+      u32x2 w;
+      w[0] = (uint32_t)f2bf(o[i][4 * g4] * inv) | ((uint32_t)f2bf(o[i][4 * g4 + 1] * inv) << 16);
+      w[1] = (uint32_t)f2bf(o[i][4 * g4 + 2] * inv) | ((uint32_t)f2bf(o[i][4 * g4 + 3] * inv) << 16);
+      *reinterpret_cast<u32x2*>(op + i * 32 + 8 * g4 + 4 * (lane >> 5)) = w;
+    }
+}
+
+// Queries that one wave of seq_kernel holds: 8 of a window of one chunk (32 or
+// 64 keys), 4 where it loops over chunks (each waits for its rows).
+bool one_chunk(const HierFrameAttnArgs& a) { return a.Lk <= 8 * (512 / a.D); }
+int query_groups(const HierFrameAttnArgs& a) { return one_chunk(a) ? (a.Lq + 7) / 8 : (a.Lq + 3) / 4; }
+// tile_kernel costs a sequence the same from 1 to 32 queries.  Windows of one
+// chunk (2,200 x 24 heads, 24 keys, D = 128), seq_kernel / tile_kernel: 8
+// queries 181 / 415 us, 16 317 / 445, 32 623 / 499.  Longer (40 x 24 heads, 200
+// keys): 3 21 / 30 us, 5 28 / 30, 8 33 / 30; 8 heads, 1,000 keys: 5 59 / 37.
+bool use_seq(const HierFrameAttnArgs& a) { return a.Lq <= (one_chunk(a) ? 16 : 4); }
+
+template <int D, int NQ>
+void launch_seq(const HierFrameAttnArgs& a, hipStream_t st) {
+  const int nqg = query_groups(a);
+  const int64_t units = (int64_t)a.B * a.H * nqg;
+  const dim3 grid((unsigned)((units + 3) / 4)), block(256);
+  const int groups = (a.Lk + 512 / D - 1) / (512 / D);   // of 512 / D rows
+#define HIER_SEQ(G, LOOP) \
+  hipLaunchKernelGGL((seq_kernel<D, NQ, G, LOOP>), grid, block, 0, st, a, (uint32_t)nqg, (uint32_t)units)
+  if (groups <= 2) HIER_SEQ(2, false);
+  else if (groups <= 3) HIER_SEQ(3, false);
+  else if (groups <= 4) HIER_SEQ(4, false);
+  else if (groups <= 6) HIER_SEQ(6, false);
+  else if (groups <= 8) HIER_SEQ(8, false);
+  else if constexpr (NQ <= 4) HIER_SEQ(8, true);
+#undef HIER_SEQ
 }
 
 template <int D>
-__global__ __launch_bounds__(64) void frame_attn_kernel(HierFrameAttnArgs a) {
-  constexpr int LPQ = D / 8;          // lanes per query
-  constexpr int QPW = 64 / LPQ;       // queries per wave
-  // the wave's query slots run over (batch, query) pairs, so sequences with
-  // fewer queries than slots share a wave; each slot reads its own
-  // sequence's keys (slots of one sequence read the same rows)
-  const int lane = threadIdx.x;
-  const int c = lane % LPQ;
-  const int slot = blockIdx.x * QPW + lane / LPQ;
-  const int h = blockIdx.y;
-  const bool valid = slot < a.B * a.Lq;
-  const int b = valid ? slot / a.Lq : 0;
-  const int qi = valid ? slot - b * a.Lq : 0;
-  const int qs = qi;
-  const u32x4 qw = *reinterpret_cast<const u32x4*>(a.q + b * a.q_sb + qs * a.q_ss + h * a.q_sh + 8 * c);
-  const int qf = a.q_frame[qs];
-  const int qblk = qf / a.n_block;
-  const float c2 = a.scale * kLog2e;
-  const uint16_t* kb = a.k + b * a.k_sb + h * a.k_sh + 8 * c;
-  const uint16_t* vb = a.v + b * a.v_sb + h * a.v_sh + 8 * c;
-  float m = -INFINITY, l = 0.f, o[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-  // keys in groups of four: the group's rows are loaded before any is used,
-  // so each wave keeps eight 16-byte loads in flight (groups of eight
-  // measured slower)
-  constexpr int G = 4;
-  for (int j0 = 0; j0 < a.Lk; j0 += G) {
-    u32x4 kwg[G], vwg[G];
-    int kfg[G];
-#pragma unroll
-    for (int u = 0; u < G; ++u) {
-      const int j = min(j0 + u, a.Lk - 1);
-      kwg[u] = *reinterpret_cast<const u32x4*>(kb + j * a.k_ss);
-      vwg[u] = *reinterpret_cast<const u32x4*>(vb + j * a.v_ss);
-      kfg[u] = a.k_frame[j];
-    }
-#pragma unroll
-    for (int u = 0; u < G; ++u) {
-      if (j0 + u >= a.Lk) break;
-      const u32x4 kw = kwg[u], vw = vwg[u];
-      const int kf = kfg[u];
-      float s = 0.f;
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const uint32_t x = qw[e], y = kw[e];
-        s = __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2, x),
-                                            __builtin_bit_cast(bf16x2, y), s, false);
-      }
-#pragma unroll
-      for (int d = 1; d < LPQ; d <<= 1) s += __shfl_xor(s, d, 64);
-      const bool vis =
-          valid && kf / a.n_block <= qblk && (a.local_attn < 0 || qf - kf < a.local_attn);
-      if (vis) {
-        const float t = s * c2;
-        const float mn = fmaxf(m, t);
-        const float alpha = __builtin_amdgcn_exp2f(m - mn);   // m = -inf: 0
-        const float p = __builtin_amdgcn_exp2f(t - mn);
-        l = l * alpha + p;
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const uint32_t w = vw[e];
-          o[2 * e] = fmaf(p, lo(w), o[2 * e] * alpha);
-          o[2 * e + 1] = fmaf(p, hi(w), o[2 * e + 1] * alpha);
-        }
-        m = mn;
-      }
-    }
+void launch_seq_d(const HierFrameAttnArgs& a, hipStream_t st) {
+  const int nqg = query_groups(a);
+  switch ((a.Lq + nqg - 1) / nqg) {
+    case 1: return launch_seq<D, 1>(a, st);
+    case 2: return launch_seq<D, 2>(a, st);
+    case 3: return launch_seq<D, 3>(a, st);
+    case 4: return launch_seq<D, 4>(a, st);
+    case 5:
+    case 6: return launch_seq<D, 6>(a, st);
+    default: return launch_seq<D, 8>(a, st);
   }
-  if (!valid) return;
-  const float inv = l > 0.f ? 1.f / l : 0.f;
-  u32x4 ow;
-#pragma unroll
-  for (int e = 0; e < 4; ++e) ow[e] = f2bf(o[2 * e] * inv) | (f2bf(o[2 * e + 1] * inv) << 16);
-  *reinterpret_cast<u32x4*>(a.o + b * a.o_sb + qi * a.o_ss + h * a.o_sh + 8 * c) = ow;
 }
 
 }  // namespace
@@ -119,13 +434,19 @@ extern "C" int hier_frame_attn(const HierFrameAttnArgs* args, void* stream) {
                    a.v_sh % 8 == 0 && a.o_sb % 8 == 0 && a.o_ss % 8 == 0 && a.o_sh % 8 == 0,
                HIER_EINVAL, "strides must keep 16-byte rows aligned");
   HIER_REQUIRE(a.H <= 65535, HIER_EUNSUPPORTED, "at most 65535 heads");
-  const int qpw = 64 / (a.D / 8);
-  const int64_t slots = (int64_t)a.B * a.Lq;
-  HIER_REQUIRE(slots / qpw < (1ll << 31) - 1, HIER_EUNSUPPORTED, "too many queries");
-  const dim3 grid((unsigned)((slots + qpw - 1) / qpw), a.H, 1);
+  const int64_t q_tiles = ((int64_t)a.Lq + 127) / 128;
+  const int64_t wgs = (int64_t)a.B * a.H * (use_seq(a) ? query_groups(a) : q_tiles);
+  HIER_REQUIRE(wgs <= hier::kMaxLaunchItems, HIER_EUNSUPPORTED, "too many queries");
+  const hipStream_t st = (hipStream_t)stream;
+  if (use_seq(a)) {
+    if (a.D == 128) launch_seq_d<128>(a, st);
+    else launch_seq_d<64>(a, st);
+    return hier::check_launch("seq_kernel");
+  }
+  const dim3 grid((unsigned)hier::xcd_grid(wgs));
   if (a.D == 128)
-    hipLaunchKernelGGL(frame_attn_kernel<128>, grid, dim3(64), 0, (hipStream_t)stream, a);
+    hipLaunchKernelGGL(tile_kernel<128>, grid, dim3(256), 0, st, a, (int)q_tiles, (int)wgs);
   else
-    hipLaunchKernelGGL(frame_attn_kernel<64>, grid, dim3(64), 0, (hipStream_t)stream, a);
-  return hier::check_launch("frame_attn_kernel");
+    hipLaunchKernelGGL(tile_kernel<64>, grid, dim3(256), 0, st, a, (int)q_tiles, (int)wgs);
+  return hier::check_launch("tile_kernel");
 }

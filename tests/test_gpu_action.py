@@ -44,6 +44,44 @@ def test_frame_attention_matches_oracle(D, local_attn):
         assert mx <= MAX_ABS and mn <= MEAN_ABS
 
 
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("Lq", [1, 2, 3, 4, 5, 8, 9, 16, 17, 32, 33, 129])
+def test_frame_attention_edges(D, Lq):
+    """Every kernel variant (waves of 1-8 queries, matrix tiles above) at
+    the edges of its key chunks and tiles, with keys that no query, one query
+    or all queries see, head counts that leave waves of a workgroup empty, and
+    q / k / v as slices of larger tensors (heads before tokens for k),
+    against float64.  Scores, weights and sums are fp32, so a result is off
+    by its own bf16 rounding (2^-9 of it) and fp32 terms far below 1e-3 of the
+    values' size."""
+    need_gpu()
+    g = torch.Generator().manual_seed(100 * D + Lq)
+    n_block = 3
+    for B, H, Lk, W in ((3, 5, 1, -1), (2, 4, 24, 21), (1, 3, 31, 4), (2, 2, 33, 6), (1, 1, 64, -1),
+                        (2, 3, 65, 9), (1, 2, 200, 30)):
+        say("frame attention edges", D, Lq, B, H, Lk, W)
+        q = torch.randn(B, Lq + 2, H + 1, D, generator=g).to(torch.bfloat16)[:, 1:-1, 1:]
+        k = torch.randn(B, H, Lk, D, generator=g).to(torch.bfloat16).transpose(1, 2)
+        v = torch.randn(B, Lk, 2 * H, D, generator=g).to(torch.bfloat16)[:, :, :H]
+        kf = torch.sort(torch.randint(0, 40, (Lk,), generator=g)).values
+        qf = 12 + torch.arange(Lq) % 20
+        qd, vd = (torch.zeros(t.shape[0], t.shape[1] + 2, 2 * H, D, dtype=torch.bfloat16,
+                              device="cuda")[:, 1:-1, :H] for t in (q, v))
+        qd.copy_(q), vd.copy_(v)
+        kd = k.transpose(1, 2).contiguous().cuda().transpose(1, 2)
+        got = frame_attention(qd, kd, vd, qf, kf, n_block, W)
+        torch.cuda.synchronize()
+        m = (kf[None] // n_block) <= (qf[:, None] // n_block)
+        if W != -1:
+            m &= qf[:, None] - kf[None] < W
+        sc = torch.einsum("bihd,bjhd->bhij", q.double(), k.double()) / math.sqrt(D)
+        p = torch.softmax(sc.masked_fill(~m, -math.inf), -1).nan_to_num(0.0)
+        ref = torch.einsum("bhij,bjhd->bihd", p, v.double())
+        err = (got.double().cpu() - ref).abs()
+        assert (err <= 2.0 ** -8 * ref.abs() + 1e-3).all(), float(err.max())
+        assert (got.cpu()[:, ~m.any(1)] == 0).all()
+
+
 class _Attn(nn.Module):
     """The attributes the reference's cached action attention reads."""
 
