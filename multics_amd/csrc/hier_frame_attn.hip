@@ -14,8 +14,8 @@
 //               lanes per row, up to 8 groups of rows: 8 KB each of K and V),
 //               scores them for every query from registers and adds the row
 //               groups' sums at the end.  2,200 sequences x 24 heads of 128,
-//               3 x 24 keys: 128-136 us, 5.2-5.5 TB/s (155 us, 4.5 TB/s, when
-//               each query read the rows for itself, four keys at a time).
+//               3 x 24 keys: 115 us, 6.1 TB/s (155 us, 4.5 TB/s, when each
+//               query read the rows for itself, four keys at a time).
 // tile_kernel   more (the keyboard branch: 660 video tokens against 96 keyboard
 //               tokens per player): 128 queries per workgroup on the matrix
 //               cores, 64-key tiles of K and V in LDS, the next tile's rows
@@ -97,17 +97,22 @@ __global__ __launch_bounds__(256, LOOP || NQ > 4 ? 2 : 3) void seq_kernel(HierFr
   const uint16_t* const vr = vb + (int64_t)r * a.v_ss;
   u32x4 k[G], v[G];
   int kf[G];
+  // a row is read once, by one wave: past the caches (the temporal branch 132 us
+  // without, 115 with); in a loop the rows' neighbours follow (1,000 keys: 34 / 47)
+  auto load = [&](const uint16_t* p) {
+    const u32x4* w = reinterpret_cast<const u32x4*>(p);
+    if constexpr (LOOP) return *w;
+    else return __builtin_nontemporal_load(w);
+  };
   auto fetch = [&](int j0) {          // a chunk's rows, all before any is used
 #pragma unroll
     for (int g = 0; g < G; ++g)
-      k[g] = *reinterpret_cast<const u32x4*>(
-          j0 + g * R + r < a.Lk ? kr + (int64_t)(j0 + g * R) * a.k_ss : kl);
+      k[g] = load(j0 + g * R + r < a.Lk ? kr + (int64_t)(j0 + g * R) * a.k_ss : kl);
 #pragma unroll
     for (int g = 0; g < G; ++g) kf[g] = a.k_frame[min(j0 + g * R + r, a.Lk - 1)];
 #pragma unroll
     for (int g = 0; g < G; ++g)
-      v[g] = *reinterpret_cast<const u32x4*>(
-          j0 + g * R + r < a.Lk ? vr + (int64_t)(j0 + g * R) * a.v_ss : vl);
+      v[g] = load(j0 + g * R + r < a.Lk ? vr + (int64_t)(j0 + g * R) * a.v_ss : vl);
   };
   u32x4 q[NQ];
 #pragma unroll
