@@ -23,7 +23,7 @@ from .rolling import rolling_cache_append  # noqa: F401  (re-exported)
 
 
 def _stream(dev) -> C.c_void_p:
-    return C.c_void_p(torch.cuda.current_stream(dev).cuda_stream)
+    return C.c_void_p(_capi.stream_of(dev))
 
 
 def ensure_action_cache(parent: dict, name: str, batch: int, n_heads: int, head_dim: int,

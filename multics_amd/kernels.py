@@ -21,7 +21,7 @@ from .metadata import HierTiledBlockLayout, TileList, backward_lists, folded_key
 
 
 def _stream(dev) -> C.c_void_p:
-    return C.c_void_p(torch.cuda.current_stream(dev).cuda_stream)
+    return C.c_void_p(_capi.stream_of(dev))
 
 
 def _rows_view(t: torch.Tensor):

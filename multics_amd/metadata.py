@@ -689,7 +689,7 @@ def build(topo: BlockTopology, device, *, segmented_block_m: Optional[int] = Non
     P, N, n, B = topo.P, topo.N, topo.n_frames, topo.B
     NS = P + N + 1
     t, dv = _topo_struct(topo, dev)
-    stream = C.c_void_p(torch.cuda.current_stream(dev).cuda_stream)
+    stream = C.c_void_p(_capi.stream_of(dev))
 
     n_seg = topo.n_seg
     # the five count arrays in one buffer: one fill, one readback
@@ -1117,7 +1117,7 @@ def ste_classes(tiles: TileList, ste_geometry):
     cls = torch.empty(max(n, 4), dtype=torch.int32, device=tiles.items.device)
     first = torch.empty(max(tiles.n_items, 1), dtype=torch.int32, device=tiles.items.device)
     _capi.call("hier_derive_ste_classes", C.byref(a), cls.data_ptr(), first.data_ptr(),
-               torch.cuda.current_stream(tiles.items.device).cuda_stream)
+               _capi.stream_of(tiles.items.device))
     cache[key] = (cls, first)
     return cache[key]
 
@@ -1152,7 +1152,7 @@ def _derive_device(tiles: TileList, ste_geometry):
     ws = torch.empty(max(ws_bytes, 1), dtype=torch.uint8, device=dev)
     totals = torch.zeros(8, dtype=torch.int64, device=dev)
     a.ws, a.ws_bytes, a.totals = ws.data_ptr(), ws_bytes, totals.data_ptr()
-    stream = torch.cuda.current_stream(dev).cuda_stream
+    stream = _capi.stream_of(dev)
     _capi.call("hier_derive_count", C.byref(a), stream)
     n_key, pairs, n_ste, n_ste_items, err = (int(x) for x in totals[:5].cpu())
     for bit, msg in _DERIVE_ERRORS:
@@ -1248,7 +1248,7 @@ def folded_key_list(tiles: TileList, kt: TileList) -> TileList:
         items=kt.items.data_ptr(), kv_idx=kv_idx.data_ptr(), kv_mask=kv_mask.data_ptr(),
         blk_and=blk.data_ptr(), acc=acc.data_ptr(), **{k: v.data_ptr() for k, v in d.items()},
         out_items=out.data_ptr())
-    _capi.call("hier_merge_hub_lists", C.byref(a), torch.cuda.current_stream(dev).cuda_stream)
+    _capi.call("hier_merge_hub_lists", C.byref(a), _capi.stream_of(dev))
     keep = torch.tensor([i for i in range(kt.n_items) if i not in drop], dtype=torch.int64,
                         device=dev)
     items = torch.cat([out[:int(item_off[-1])], kt.items[:kt.n_items].index_select(0, keep)])
@@ -1292,7 +1292,7 @@ def _trim_items(items: torch.Tensor, n: int, kv_mask: torch.Tensor,
     a = _capi.HierTrimArgs(n_items=n, items=items.data_ptr(), kv_mask=kv_mask.data_ptr(),
                            row_table=None if row_table is None else row_table.data_ptr(),
                            out_items=out.data_ptr())
-    _capi.call("hier_trim_key_lists", C.byref(a), torch.cuda.current_stream(items.device).cuda_stream)
+    _capi.call("hier_trim_key_lists", C.byref(a), _capi.stream_of(items.device))
     return out
 
 
@@ -1573,7 +1573,7 @@ class MembershipLogitsPlan:
         if tuple(logits.shape) != (T, N, P):
             raise ValueError(f"membership logits must be [T,N,P] = {(T, N, P)}")
         lg = logits.detach().to(device=dev, dtype=torch.float32).contiguous()
-        stream = torch.cuda.current_stream(dev).cuda_stream
+        stream = _capi.stream_of(dev)
         self._margs.logits = lg.data_ptr()
         _capi.call("hier_membership_from_logits", C.byref(self._margs), stream)
         sup = self.sup
@@ -1662,6 +1662,33 @@ def cached_tiles(*, device, P, N, L, KL, KG, n_frames, n_block, local_attn, fram
             labels=labels, q_active=q_active, direct_player=direct_player, membership=membership,
             global_only=global_only, hier_no_local_hub=no_local, tile_bases=tile_bases)
         hit = build(topo, device).tiles
+        _lru_put(_META_CACHE, key, hit, "WAN_HIER_SEGMENTED_META_CACHE_SIZE", "64")
+    return hit
+
+
+def cached_window_tiles(cache, end_frame: int, *, device, n_frames, n_block, local_attn, labels,
+                        q_active, direct_player, membership=None, global_only=None,
+                        hier_no_local_hub=False) -> TileList:
+    """``cached_tiles`` over the window that a ``HierPagedKVCache`` holds for a
+    block ending at ``end_frame``.  The list is kept under what the window is
+    made of -- the cache's shape, its ring and its local-hub flags -- beside the
+    block's topology (host arrays), in the same LRU, so the later passes over a
+    block neither gather its pages nor hash them."""
+    raw = lambda x: None if x is None else (np.shape(x), np.asarray(x).tobytes())
+    key = ("window", str(device), cache.P, cache.N, cache.L, cache.KL, cache.KG, cache.R,
+           cache.no_local, int(end_frame), cache.slot_frame.tobytes(),
+           cache.local_active.tobytes(), n_frames, n_block, local_attn, raw(labels), raw(q_active),
+           bool(direct_player), bool(hier_no_local_hub), raw(membership), raw(global_only))
+    hit = _lru_get(_META_CACHE, key)
+    if hit is None:
+        frames, bases, lact = cache.window(end_frame)
+        listed = lambda x: None if x is None else np.asarray(x).tolist()
+        hit = cached_tiles(
+            device=device, P=cache.P, N=cache.N, L=cache.L, KL=cache.KL, KG=cache.KG,
+            n_frames=n_frames, n_block=n_block, local_attn=local_attn, frames=frames,
+            tile_bases=bases, local_active_frames=lact, labels=listed(labels),
+            q_active=listed(q_active), direct_player=direct_player, membership=membership,
+            global_only=global_only, hier_no_local_hub=hier_no_local_hub)
         _lru_put(_META_CACHE, key, hit, "WAN_HIER_SEGMENTED_META_CACHE_SIZE", "64")
     return hit
 

@@ -34,7 +34,7 @@ import torch.nn as nn
 import torch.nn.functional as F
 
 from . import metadata as M
-from .kernels import (_covers_all_rows, _uncleared, gated_residual, hier_attention,
+from .kernels import (_uncleared, gated_residual, hier_attention,
                       hier_attention_forward, qk_prologue_train, qkv_prologue)
 from .hier_masks import HierBlockMask
 from .kv_cache import stream_pool
@@ -92,10 +92,10 @@ def rope_apply(x: torch.Tensor, freqs: torch.Tensor, num_heads: int) -> torch.Te
 
 
 def _attn_out(tiles, s, H, D, device):
-    """Output buffer of a full-sequence forward: uncleared when the list's
-    items own every one of the s rows (the kernel then writes each, 0 for a
-    row that sees no key), zero-filled otherwise."""
-    if _covers_all_rows(tiles) and tiles.row_extent == s:
+    """Output buffer of a forward: uncleared when the list's items own every
+    one of the s rows (the kernel then writes each, 0 for a row that sees no
+    key), zero-filled otherwise."""
+    if tiles.rows_exact_cover and tiles.row_extent == s:
         return _uncleared(size=(s, H, D), dtype=torch.bfloat16, device=device)
     return torch.zeros((s, H, D), dtype=torch.bfloat16, device=device)
 
@@ -422,10 +422,9 @@ class SelfAttention(nn.Module):
             if start_frame < 0 or start_frame + n > T_full:
                 raise ValueError(f"hier_hub membership T={T_full} does not cover cached block "
                                  f"[{start_frame},{start_frame + n})")
-            mb = mem[start_frame:start_frame + n]
-            gb = go[start_frame:start_frame + n]
-            if n > 1 and (not torch.equal(mb, mb[:1].expand_as(mb)) or
-                          not torch.equal(gb, gb[:1].expand_as(gb))):
+            mb = mem[start_frame:start_frame + n].numpy()
+            gb = go[start_frame:start_frame + n].numpy()
+            if n > 1 and ((mb[1:] != mb[:1]).any() or (gb[1:] != gb[:1]).any()):
                 raise ValueError("hier_hub cached inference requires membership / global_only "
                                  "constant inside each latent block")
             act = act[start_frame:start_frame + n]
@@ -444,16 +443,13 @@ class SelfAttention(nn.Module):
             q, k, v = (torch.stack([pt[j] for pt in parts], dim=1).view(s, b * H, D)
                        for j in range(3))
         kv_cache.append(k, v, start_frame, n, act.numpy())
-        frames, bases, lact = kv_cache.window(start_frame + n - 1)
-        tiles = M.cached_tiles(
-            device=x.device, P=P, N=N, L=L, KL=KL, KG=KG, n_frames=n,
+        tiles = M.cached_window_tiles(
+            kv_cache, start_frame + n - 1, device=x.device, n_frames=n,
             n_block=int(self.num_frame_per_block), local_attn=int(self.local_attn_size),
-            frames=frames, tile_bases=bases, local_active_frames=lact,
-            labels=None if labels is None else labels.tolist(), q_active=act.tolist(),
-            direct_player=bool(direct_player),
-            membership=mem.numpy() if use_mem else None,
+            labels=None if labels is None else labels.numpy(), q_active=act.numpy(),
+            direct_player=bool(direct_player), membership=mem.numpy() if use_mem else None,
             global_only=go.numpy() if use_mem else None, hier_no_local_hub=no_local)
-        out = torch.zeros((s, b * H, D), dtype=torch.bfloat16, device=x.device)
+        out = _attn_out(tiles, s, b * H, D, x.device)
         hier_attention_forward(q, kv_cache.k, kv_cache.v, tiles, out)
         out = out.view(s, b, dim).transpose(0, 1)
         return self.o(out.to(self.o.weight.dtype))

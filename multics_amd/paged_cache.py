@@ -33,7 +33,7 @@ from . import _capi
 
 
 def _stream(dev) -> C.c_void_p:
-    return C.c_void_p(torch.cuda.current_stream(dev).cuda_stream)
+    return C.c_void_p(_capi.stream_of(dev))
 
 
 class HierPagedKVCache:

@@ -136,6 +136,52 @@ def test_module_rollout_matches_cached_oracle(case, store):
             assert mx <= MAX_ABS and mn <= MEAN_ABS
 
 
+@pytest.mark.parametrize("case", CASES, ids=[c[0] for c in CASES])
+def test_rollout_output_is_written_whole(case, monkeypatch):
+    """A block's output buffer is left uncleared where its list's items own
+    every row; pre-filled with NaN, the rollout (inactive hub slots among the
+    membership case's) still matches the oracle in every row."""
+    from multics_amd import kernels
+    monkeypatch.setattr(kernels, "_UNCLEARED_FILL", float("nan"))
+    test_module_rollout_matches_cached_oracle(case, "paged")
+
+
+def test_window_lists_follow_the_cache():
+    """Lists kept per window: the same frames in another ring order or with
+    other local-hub flags are another window, an equal cache shares the list."""
+    need_gpu()
+    kw = dict(num_players=2, num_groups=2, num_patches=8, num_local_hub_tokens=2,
+              num_global_hub_tokens=1, num_heads=1, head_dim=64, local_attn_size=3,
+              num_frame_per_block=3, device="cuda")
+    S = 2 * 3 * 8 + 3 * (2 * 2 + 1)
+    blk = torch.zeros(S, 1, 64, dtype=torch.bfloat16, device="cuda")
+    act = np.array([[True, True]] * 3)
+
+    def tiles(starts, flags=act):
+        c = HierPagedKVCache(**kw)
+        for f in starts:
+            c.append(blk, blk, f, 3, flags if f == starts[-1] else act)
+        t = M.cached_window_tiles(c, starts[-1] + 2, device=blk.device, n_frames=3, n_block=3,
+                                  local_attn=3, labels=np.zeros((3, 2), np.int64), q_active=act,
+                                  direct_player=True)
+        frames, bases, lact = c.window(starts[-1] + 2)
+        want = M.cached_tiles(device=blk.device, P=2, N=2, L=8, KL=2, KG=1, n_frames=3, n_block=3,
+                              local_attn=3, frames=frames, tile_bases=bases,
+                              local_active_frames=lact, labels=np.zeros((3, 2), int).tolist(),
+                              q_active=act.tolist(), direct_player=True)
+        assert torch.equal(t.kv_idx, want.kv_idx) and torch.equal(t.kv_mask, want.kv_mask)
+        assert torch.equal(t.items, want.items)
+        return t
+
+    say("window lists")
+    a = tiles([0, 3])
+    assert tiles([0, 3]) is a
+    assert tiles([3]) is not a and tiles([3, 6]) is not a
+    off = act.copy()
+    off[1, 1] = False
+    assert tiles([0, 3], off) is not a
+
+
 def test_reference_cached_backend_call():
     """The plugin keyword call on per-stream windows taken from the oracle's caches."""
     need_gpu()
