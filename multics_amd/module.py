@@ -205,7 +205,9 @@ class SelfAttention(nn.Module):
         dim = H * D
         if self._fused_ok(x, cam_tokens) and dim % 512 == 0 and dim <= 4096:
             cam = self._check_cam(x, cam_tokens)
-            qx, kx, vx = (lin(x)[0] for lin in (self.q, self.k, self.v))
+            # (views of the [1, s, dim] projections: the backward of an index
+            # would copy each gradient into a cleared buffer)
+            qx, kx, vx = (lin(x).view(s, dim) for lin in (self.q, self.k, self.v))
             cs, sn = freqs_to_cos_sin(freqs, device=x.device)
             q, k = qk_prologue_train(
                 qx, kx, norm_q_w=self.norm_q.weight, norm_k_w=self.norm_k.weight, rope_cos=cs,
