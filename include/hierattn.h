@@ -171,7 +171,7 @@ typedef struct HierDeriveArgs {
 
 /* Workspace bytes for the sizes in args (ws may be NULL); -1 on NULL args.  */
 int64_t hier_derive_workspace(const HierDeriveArgs* args);
-/* Pass 1: groups, token map, run table, list sizes and offsets -> totals.   */
+/* Pass 1: groups, token map, run table, list sizes -> totals.               */
 int hier_derive_count(const HierDeriveArgs* args, void* stream);
 /* Pass 2: the two lists, their per-64 mask ANDs and their items.            */
 int hier_derive_build(const HierDeriveArgs* args, void* stream);
@@ -248,6 +248,8 @@ typedef struct HierTrimArgs {
 } HierTrimArgs;
 
 int hier_trim_key_lists(const HierTrimArgs* args, void* stream);
+/* Two lists in one launch (n_items = 0: none). */
+int hier_trim_key_lists2(const HierTrimArgs* a, const HierTrimArgs* b, void* stream);
 
 /* Membership-dependent topology arrays of a full-sequence membership        */
 /* topology from soft membership logits, in one launch: membership =        */
@@ -490,6 +492,9 @@ typedef struct HierSteReduceArgs {
 } HierSteReduceArgs;
 
 int hier_ste_reduce(const HierSteReduceArgs* args, void* stream);
+/* The same times sigmoid'(logits[t][g][p]) (fp32): the straight-through      */
+/* gradient of the membership logits.                                        */
+int hier_ste_logit_grad(const HierSteReduceArgs* args, const float* logits, void* stream);
 
 /* ------------------------------------------------------------------------ */
 /* Paged KV cache append: copy the new K/V rows of a cached block into their */

@@ -172,6 +172,7 @@ EXPORTS = {
     "hier_membership_from_logits": [C.POINTER(HierMembershipArgs), vp],
     "hier_merge_hub_lists": [C.POINTER(HierMergeArgs), vp],
     "hier_trim_key_lists": [C.POINTER(HierTrimArgs), vp],
+    "hier_trim_key_lists2": [C.POINTER(HierTrimArgs), C.POINTER(HierTrimArgs), vp],
     "hier_qkv_prologue": [C.POINTER(HierPrologueArgs), vp],
     "hier_qk_prologue_bwd_waves": [C.POINTER(HierPrologueBwdArgs)],
     "hier_qk_prologue_bwd": [C.POINTER(HierPrologueBwdArgs), vp],
@@ -180,6 +181,7 @@ EXPORTS = {
     "hier_attn_bwd": [C.POINTER(HierBwdArgs), vp],
     "hier_attn_bwd_noalloc": [C.POINTER(HierBwdArgs), vp],
     "hier_ste_reduce": [C.POINTER(HierSteReduceArgs), vp],
+    "hier_ste_logit_grad": [C.POINTER(HierSteReduceArgs), vp, vp],
     "hier_kv_append": [C.POINTER(HierPageArgs), vp],
     "hier_frame_attn": [C.POINTER(HierFrameAttnArgs), vp],
     "hier_gated_residual": [C.POINTER(HierGateArgs), vp],

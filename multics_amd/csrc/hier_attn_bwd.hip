@@ -1227,7 +1227,9 @@ extern "C" int hier_attn_bwd_noalloc(const HierBwdArgs* args, void* stream) {
 // fixed-order tree in LDS: deterministic.
 namespace {
 
-__global__ __launch_bounds__(256) void ste_reduce_kernel(HierSteReduceArgs a) {
+// With `logits` the result is the logits' straight-through gradient,
+// sigmoid'(logit) times the sum.
+__global__ __launch_bounds__(256) void ste_reduce_kernel(HierSteReduceArgs a, const float* logits) {
   __shared__ float part[256];
   const int o = blockIdx.x;
   const int p = o % a.P, g = (o / a.P) % a.N, t = o / (a.P * a.N);
@@ -1249,13 +1251,18 @@ __global__ __launch_bounds__(256) void ste_reduce_kernel(HierSteReduceArgs a) {
     if (threadIdx.x < w) part[threadIdx.x] += part[threadIdx.x + w];
     __syncthreads();
   }
-  if (threadIdx.x == 0) a.out[o] = part[0];
+  if (threadIdx.x != 0) return;
+  float r = part[0];
+  if (logits != nullptr) {
+    const float sig = 1.f / (1.f + expf(-logits[o]));
+    r *= sig * (1.f - sig);
+  }
+  a.out[o] = r;
 }
 
 }  // namespace
 
-extern "C" int hier_ste_reduce(const HierSteReduceArgs* args, void* stream) {
-  hier::clear_error();
+static int ste_reduce(const HierSteReduceArgs* args, const float* logits, void* stream) {
   HIER_REQUIRE(args != nullptr, HIER_EINVAL, "args is NULL");
   const HierSteReduceArgs& a = *args;
   HIER_REQUIRE(a.H >= 1 && a.P >= 1 && a.T >= 1 && a.L >= 1 && a.N >= 1 && a.KL >= 0 &&
@@ -1275,6 +1282,18 @@ extern "C" int hier_ste_reduce(const HierSteReduceArgs* args, void* stream) {
   const int64_t n_out = (int64_t)a.T * a.N * a.P;
   HIER_REQUIRE(n_out <= INT32_MAX, HIER_EUNSUPPORTED, "too many outputs");
   hipLaunchKernelGGL(ste_reduce_kernel, dim3((unsigned)n_out), dim3(256), 0, (hipStream_t)stream,
-                     a);
+                     a, logits);
   return hier::check_launch("ste_reduce_kernel");
+}
+
+extern "C" int hier_ste_reduce(const HierSteReduceArgs* args, void* stream) {
+  hier::clear_error();
+  return ste_reduce(args, nullptr, stream);
+}
+
+extern "C" int hier_ste_logit_grad(const HierSteReduceArgs* args, const float* logits,
+                                   void* stream) {
+  hier::clear_error();
+  HIER_REQUIRE(logits != nullptr, HIER_EINVAL, "logits is NULL");
+  return ste_reduce(args, logits, stream);
 }

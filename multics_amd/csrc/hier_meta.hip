@@ -649,9 +649,18 @@ extern "C" int hier_meta_build(const HierTopo* topo, const HierMetaOut* out, voi
 //
 // Pass 1 (hier_derive_count) maps tokens to groups, collects the runs into a
 // dense [key group][query group][query frame] table of key-frame bitmasks,
-// counts both lists and prefix-sums their offsets; the caller reads back the
-// totals (entries, pairs, error flags) to size pass 2 (hier_derive_build),
-// which writes the lists, the per-64-key ANDs of the masks and the items.
+// counts both lists and prefix-sums the STE list's offsets; the caller reads
+// back the totals (entries, pairs, error flags) to size pass 2
+// (hier_derive_build), which writes the lists, the per-64-key ANDs of the masks
+// and the items.  A list whose membership changes is rebuilt every training
+// step, and each pass is a few microseconds of launch and latency, so what
+// bounds the chain is its launches: the fills and the groups share one, the
+// key-major offsets, ANDs and items are written by the workgroup that writes
+// the list, and the STE passes run only with an STE geometry.  With the two
+// lists cut in one launch (hier_trim_key_lists2) and the logits' gradient in
+// the STE reduction's (hier_ste_logit_grad), a training step of 4 players, 9
+// frames of 40 tokens, 8 heads went from 219 to 170 us, one of 8 players, 18
+// frames of 60, 12 heads from 812 to 774 us.
 
 namespace {
 
@@ -677,7 +686,6 @@ struct DeriveWs {
   uint32_t* table;        // [n_groups][n_groups][nq]: (key group G, query group g, frame j)
   int32_t* runs;          // [n_groups][n_groups][nq]: runs of (query g, key group G, key frame f)
   int32_t* t_size;        // [n_groups] padded key-major list sizes
-  int64_t* t_off;         // [n_groups + 1]
   int32_t* s_cnt;         // [n_groups][kClasses]
   int32_t* s_size;        // [n_groups] padded STE list sizes
   int64_t* s_off;         // [n_groups + 1]
@@ -699,7 +707,6 @@ __host__ __device__ inline int64_t derive_ws_layout(const HierDeriveArgs& a, Der
   d.table = reinterpret_cast<uint32_t*>(take(4 * tab));
   d.runs = reinterpret_cast<int32_t*>(take(4 * tab));
   d.t_size = reinterpret_cast<int32_t*>(take(4 * ng));
-  d.t_off = reinterpret_cast<int64_t*>(take(8 * (ng + 1)));
   d.s_cnt = reinterpret_cast<int32_t*>(take(4 * ng * kClasses));
   d.s_size = reinterpret_cast<int32_t*>(take(4 * ng));
   d.s_off = reinterpret_cast<int64_t*>(take(8 * (ng + 1)));
@@ -726,19 +733,6 @@ __global__ void derive_fill_kernel(int32_t* p, int64_t n, int32_t v) {
     p[i] = v;
 }
 
-// Up to four fills in one launch (blockIdx.y selects the array).
-struct FillJobs {
-  int32_t* p[4];
-  int64_t n[4];
-  int32_t v[4];
-};
-__global__ void derive_fill4_kernel(FillJobs f) {
-  const int j = blockIdx.y;
-  for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < f.n[j];
-       i += (int64_t)gridDim.x * blockDim.x)
-    f.p[j][i] = f.v[j];
-}
-
 // Block-wide exclusive scan of one value per thread (kScanThreads threads).
 __device__ int64_t block_scan(int64_t v, int64_t* sh, int64_t* total) {
   const int t = threadIdx.x;
@@ -756,12 +750,28 @@ __device__ int64_t block_scan(int64_t v, int64_t* sh, int64_t* total) {
   return incl - v;
 }
 
-// Groups: item i starts a group when its row_start is 0; grp_first[n_groups]
-// = n_items.  Totals zeroed.
-__global__ __launch_bounds__(kScanThreads) void derive_groups_kernel(HierDeriveArgs a, DeriveWs w) {
+// First launch of pass 1.  blockIdx.y = 0 .. 2: tok_g cleared to -1, table and
+// runs to 0.  Workgroup (0, 3): the groups -- item i starts a group when its
+// row_start is 0; grp_first[n_groups] = n_items -- and the totals zeroed.
+// (Independent work in one launch: each of these passes is a few
+// microseconds of latency.)
+__global__ __launch_bounds__(kScanThreads) void derive_init_kernel(HierDeriveArgs a, DeriveWs w) {
   __shared__ int64_t sh[kScanThreads];
   const int t = threadIdx.x;
+  if (blockIdx.y < 3) {
+    const int64_t tab = (int64_t)a.n_groups * a.n_groups * a.nq_max;
+    int32_t* p = blockIdx.y == 0 ? w.tok_g
+                                 : blockIdx.y == 1 ? reinterpret_cast<int32_t*>(w.table) : w.runs;
+    const int64_t n = blockIdx.y == 0 ? a.rows : tab;
+    const int32_t v = blockIdx.y == 0 ? -1 : 0;
+    for (int64_t i = blockIdx.x * (int64_t)kScanThreads + t; i < n;
+         i += (int64_t)gridDim.x * kScanThreads)
+      p[i] = v;
+    return;
+  }
+  if (blockIdx.x != 0) return;
   if (t < 8) a.totals[t] = 0;
+  for (int g = t; g <= a.n_groups; g += kScanThreads) w.grp_first[g] = 0;
   __syncthreads();
   if (t == 0 && (a.n_items < 1 || a.items[3] != 0)) flag(a.totals, kErrItems);
   int64_t carry = 0;
@@ -792,7 +802,7 @@ struct GroupDesc {
 };
 
 // A group's descriptor, from its first item; the key range is clamped to the
-// list (an item outside it is flagged by derive_groups_kernel).
+// list (an item outside it is flagged by derive_init_kernel).
 __device__ __forceinline__ GroupDesc group_desc(const HierDeriveArgs& a, const DeriveWs& w, int g) {
   const int32_t* it = a.items + 8 * (int64_t)w.grp_first[g];
   const int off = min(max(it[5], 0), a.kv_len);
@@ -879,7 +889,8 @@ __global__ __launch_bounds__(kDeriveThreads) void derive_runs_kernel(HierDeriveA
   }
 }
 
-// Key-major list size of key group G (padded to 64) and its (query, key) pairs.
+// Key-major list size of key group G (padded to 64) and its (query, key)
+// pairs; totals [0] entries, [1] pairs.
 __global__ __launch_bounds__(kDeriveThreads) void derive_key_sizes_kernel(HierDeriveArgs a,
                                                                           DeriveWs w) {
   __shared__ int64_t s_size, s_pairs;
@@ -904,8 +915,12 @@ __global__ __launch_bounds__(kDeriveThreads) void derive_key_sizes_kernel(HierDe
   atomicAdd(reinterpret_cast<unsigned long long*>(&s_pairs), (unsigned long long)pairs);
   __syncthreads();
   if (threadIdx.x == 0) {
-    w.t_size[G] = (int32_t)((s_size + kTileKeys - 1) / kTileKeys * kTileKeys);
+    const int64_t padded = (s_size + kTileKeys - 1) / kTileKeys * kTileKeys;
+    w.t_size[G] = (int32_t)padded;
     atomicAdd(reinterpret_cast<unsigned long long*>(&a.totals[1]), (unsigned long long)s_pairs);
+    const int64_t before = (int64_t)atomicAdd(reinterpret_cast<unsigned long long*>(&a.totals[0]),
+                                              (unsigned long long)padded);
+    if (before + padded > INT32_MAX) flag(a.totals, kErrOverflow);
   }
 }
 
@@ -980,54 +995,73 @@ __global__ __launch_bounds__(kDeriveThreads) void derive_ste_count_kernel(HierDe
   if (threadIdx.x == 0) w.s_size[g] = (n + kTileKeys - 1) / kTileKeys * kTileKeys;
 }
 
-// Offsets of both lists and of the STE items; totals [0] key-major entries,
-// [2] STE entries, [3] STE items.
+// Offsets of the STE lists and items; totals [2] STE entries, [3] STE items.
 __global__ __launch_bounds__(kScanThreads) void derive_scan_kernel(HierDeriveArgs a, DeriveWs w) {
   __shared__ int64_t sh[kScanThreads];
-  int64_t ct = 0, cs = 0, ci = 0;
+  int64_t cs = 0, ci = 0;
   for (int base = 0; base < a.n_groups; base += kScanThreads) {
     const int g = base + threadIdx.x;
     const bool in = g < a.n_groups;
-    const int64_t vt = in ? w.t_size[g] : 0, vs = in ? w.s_size[g] : 0;
+    const int64_t vs = in ? w.s_size[g] : 0;
     const int64_t vi = (in && vs > 0) ? (int64_t)(w.grp_first[g + 1] - w.grp_first[g]) : 0;
-    int64_t tt, ts, ti;
-    const int64_t et = block_scan(vt, sh, &tt);
+    int64_t ts, ti;
     const int64_t es = block_scan(vs, sh, &ts);
     const int64_t ei = block_scan(vi, sh, &ti);
     if (in) {
-      w.t_off[g] = ct + et;
       w.s_off[g] = cs + es;
       w.s_item_off[g] = ci + ei;
     }
-    ct += tt;
     cs += ts;
     ci += ti;
   }
   if (threadIdx.x == 0) {
-    w.t_off[a.n_groups] = ct;
     w.s_off[a.n_groups] = cs;
     w.s_item_off[a.n_groups] = ci;
-    a.totals[0] = ct;
     a.totals[2] = cs;
     a.totals[3] = ci;
-    if (ct > INT32_MAX || cs > INT32_MAX) flag(a.totals, kErrOverflow);
+    if (cs > INT32_MAX) flag(a.totals, kErrOverflow);
   }
 }
 
-// Key-major list of key group G: unit offsets by a block scan over the
-// (g, j) units, then every entry finds its unit by binary search.
+// Key-major list of key group G, at the sum of the sizes of the groups before
+// it: unit offsets by a block scan over the (g, j) units, then every entry
+// finds its unit by binary search.  Then the AND of the masks of every 64
+// entries, and the group's items: the forward items with the list's offset /
+// size (an empty list after a flagged pass 1, or where the list does not fit
+// the caller's size: the backward then reads nothing through them).
 __global__ __launch_bounds__(kScanThreads) void derive_key_write_kernel(HierDeriveArgs a,
                                                                         DeriveWs w) {
   __shared__ int64_t sh[kScanThreads];
   __shared__ int32_t u_off[kScanThreads];
   __shared__ int32_t u_id[kScanThreads];
-  // after a flagged pass 1 the offsets are not trusted: nothing is written
-  if (a.totals[4] != 0) return;
+  __shared__ int64_t base_s;
   const int G = blockIdx.x;
   const int ng = a.n_groups, nq = a.nq_max, nu = ng * nq;
-  const int64_t base = w.t_off[G];
   const int64_t lim = a.key_entries;   // the caller's list size bounds every store
-  const int padded = w.t_size[G];
+  // after a flagged pass 1 the offsets are not trusted: no list is written
+  const bool ok = a.totals[4] == 0;
+  if (threadIdx.x == 0) base_s = 0;
+  __syncthreads();
+  if (ok) {
+    int64_t v = 0;
+    for (int g = threadIdx.x; g < G; g += kScanThreads) v += w.t_size[g];
+    if (v != 0)
+      atomicAdd(reinterpret_cast<unsigned long long*>(&base_s), (unsigned long long)v);
+  }
+  __syncthreads();
+  const int64_t base = base_s;
+  const int padded = ok ? w.t_size[G] : 0;
+  const bool fits = ok && base + padded <= lim;
+  for (int i = threadIdx.x; i < a.n_items; i += kScanThreads)
+    if (w.grp_of_item[i] == G) {
+      const int32_t* it = a.items + 8 * (int64_t)i;
+      int32_t* o = a.key_items + 8 * (int64_t)i;
+      for (int e = 0; e < 5; ++e) o[e] = it[e];
+      o[5] = fits ? (int32_t)base : 0;
+      o[6] = fits ? padded : 0;
+      o[7] = it[7];
+    }
+  if (!ok) return;
   const uint32_t* row = w.table + (int64_t)G * nu;
   int64_t done = 0;   // entries written before this chunk of units
   for (int u0 = 0; u0 < nu; u0 += kScanThreads) {
@@ -1066,6 +1100,13 @@ __global__ __launch_bounds__(kScanThreads) void derive_key_write_kernel(HierDeri
   for (int64_t p = done + threadIdx.x; p < padded && base + p < lim; p += blockDim.x) {
     a.key_q_idx[base + p] = 0;
     a.key_q_mask[base + p] = 0;
+  }
+  __syncthreads();   // the masks are written
+  for (int t = threadIdx.x >> 6; t < padded / 64 && base + 64 * (int64_t)(t + 1) <= lim;
+       t += kScanThreads / 64) {   // one wave per tile
+    uint32_t v = a.key_q_mask[base + 64 * (int64_t)t + (threadIdx.x & 63)];
+    for (int d = 32; d >= 1; d >>= 1) v &= __shfl_xor(v, d);
+    if ((threadIdx.x & 63) == 0) a.key_blk_and[base / 64 + t] = v;
   }
 }
 
@@ -1151,20 +1192,6 @@ __global__ __launch_bounds__(kDeriveThreads) void derive_ste_write_kernel(HierDe
   }
 }
 
-// Key-major items: the forward items with their group's list offset / size.
-__global__ void derive_key_items_kernel(HierDeriveArgs a, DeriveWs w) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= a.n_items) return;
-  for (int e = 0; e < 8; ++e) a.key_items[8 * (int64_t)i + e] = a.items[8 * (int64_t)i + e];
-  // a flagged pass 1 or a list past the caller's size: an empty list (the
-  // backward then reads nothing through this item)
-  const bool ok = a.totals[4] == 0;
-  const int g = ok ? w.grp_of_item[i] : 0;
-  const bool fits = ok && w.t_off[g] + w.t_size[g] <= a.key_entries;
-  a.key_items[8 * (int64_t)i + 5] = fits ? (int32_t)w.t_off[g] : 0;
-  a.key_items[8 * (int64_t)i + 6] = fits ? w.t_size[g] : 0;
-}
-
 // AND of the masks of every 64 entries (one wave per tile).
 __global__ void derive_blk_and_kernel(const uint32_t* mask, uint32_t* blk, int64_t n_tiles) {
   const int64_t tile = blockIdx.x * (int64_t)(blockDim.x / 64) + (threadIdx.x >> 6);
@@ -1216,19 +1243,19 @@ extern "C" int hier_derive_count(const HierDeriveArgs* args, void* stream) {
   const HierDeriveArgs& a = *args;
   hipStream_t s = (hipStream_t)stream;
   const int64_t tab = (int64_t)a.n_groups * a.n_groups * a.nq_max;
-  FillJobs fj = {{w.grp_first, w.tok_g, reinterpret_cast<int32_t*>(w.table), w.runs},
-                 {(int64_t)a.n_groups + 1, a.rows, tab, tab},
-                 {0, -1, 0, 0}};
-  const int64_t fmax = std::max<int64_t>(std::max<int64_t>(a.n_groups + 1, a.rows), tab);
-  hipLaunchKernelGGL(derive_fill4_kernel, dim3((unsigned)std::min<int64_t>((fmax + 255) / 256, 1024), 4),
-                     dim3(256), 0, s, fj);
-  hipLaunchKernelGGL(derive_groups_kernel, dim3(1), dim3(kScanThreads), 0, s, a, w);
+  const int64_t fmax = std::max<int64_t>(a.rows, tab);
+  hipLaunchKernelGGL(derive_init_kernel,
+                     dim3((unsigned)std::min<int64_t>((fmax + kScanThreads - 1) / kScanThreads, 256), 4),
+                     dim3(kScanThreads), 0, s, a, w);
   hipLaunchKernelGGL(derive_tokens_kernel, dim3(a.n_groups), dim3(kDeriveThreads), 0, s, a, w);
   hipLaunchKernelGGL(derive_runs_kernel, dim3(a.n_groups, kRunSplit), dim3(kDeriveThreads), 0, s,
                      a, w);
   hipLaunchKernelGGL(derive_key_sizes_kernel, dim3(a.n_groups), dim3(kDeriveThreads), 0, s, a, w);
-  hipLaunchKernelGGL(derive_ste_count_kernel, dim3(a.n_groups), dim3(kDeriveThreads), 0, s, a, w);
-  hipLaunchKernelGGL(derive_scan_kernel, dim3(1), dim3(kScanThreads), 0, s, a, w);
+  // without an STE geometry every STE list is empty: totals [2] and [3] stay 0
+  if ((int64_t)a.P * a.T * a.L + (int64_t)a.T * a.N * a.KL > 0) {
+    hipLaunchKernelGGL(derive_ste_count_kernel, dim3(a.n_groups), dim3(kDeriveThreads), 0, s, a, w);
+    hipLaunchKernelGGL(derive_scan_kernel, dim3(1), dim3(kScanThreads), 0, s, a, w);
+  }
   return hier::check_launch("derive count kernels");
 }
 
@@ -1269,12 +1296,6 @@ extern "C" int hier_derive_build(const HierDeriveArgs* args, void* stream) {
                  HIER_EINVAL, "STE output pointer is NULL");
   hipStream_t s = (hipStream_t)stream;
   hipLaunchKernelGGL(derive_key_write_kernel, dim3(a.n_groups), dim3(kScanThreads), 0, s, a, w);
-  hipLaunchKernelGGL(derive_key_items_kernel, dim3((a.n_items + 255) / 256), dim3(256), 0, s, a,
-                     w);
-  const int64_t kt = a.key_entries / kTileKeys;
-  if (kt > 0)
-    hipLaunchKernelGGL(derive_blk_and_kernel, dim3((unsigned)((kt + 3) / 4)), dim3(256), 0, s,
-                       a.key_q_mask, a.key_blk_and, kt);
   if (ste) {
     hipLaunchKernelGGL(derive_ste_write_kernel, dim3(a.n_groups), dim3(kDeriveThreads), 0, s, a,
                        w);
@@ -1510,11 +1531,14 @@ namespace {
 
 constexpr int kTrimThreads = 256;
 
-__global__ __launch_bounds__(kTrimThreads) void trim_kernel(HierTrimArgs a) {
+// (two lists in one launch: the items of `b` follow those of `first`)
+__global__ __launch_bounds__(kTrimThreads) void trim_kernel(HierTrimArgs first, HierTrimArgs b) {
   __shared__ int32_t it[8];
   __shared__ uint32_t bits_s;
   __shared__ int first_s, last_s;
-  const int64_t i = blockIdx.x;
+  const bool second = (int)blockIdx.x >= first.n_items;
+  const HierTrimArgs& a = second ? b : first;
+  const int64_t i = second ? blockIdx.x - first.n_items : blockIdx.x;
   if (threadIdx.x < 8) it[threadIdx.x] = a.items[8 * i + threadIdx.x];
   if (threadIdx.x == 0) {
     bits_s = 0u;
@@ -1571,13 +1595,27 @@ __global__ __launch_bounds__(kTrimThreads) void trim_kernel(HierTrimArgs a) {
 
 }  // namespace
 
+static int trim_lists(const HierTrimArgs& a, const HierTrimArgs& b, void* stream) {
+  for (const HierTrimArgs* t : {&a, &b}) {
+    HIER_REQUIRE(t->n_items >= 0, HIER_EINVAL, "invalid n_items=%d", t->n_items);
+    HIER_REQUIRE(t->n_items == 0 || (t->items && t->kv_mask && t->out_items), HIER_EINVAL,
+                 "NULL pointer");
+  }
+  const int64_t n = (int64_t)a.n_items + b.n_items;
+  HIER_REQUIRE(n <= INT32_MAX, HIER_EUNSUPPORTED, "too many work items");
+  if (n == 0) return HIER_OK;
+  hipLaunchKernelGGL(trim_kernel, dim3((unsigned)n), dim3(kTrimThreads), 0, (hipStream_t)stream, a, b);
+  return hier::check_launch("trim_kernel");
+}
+
 extern "C" int hier_trim_key_lists(const HierTrimArgs* args, void* stream) {
   hier::clear_error();
   HIER_REQUIRE(args != nullptr, HIER_EINVAL, "args is NULL");
-  const HierTrimArgs& a = *args;
-  HIER_REQUIRE(a.n_items >= 0, HIER_EINVAL, "invalid n_items=%d", a.n_items);
-  if (a.n_items == 0) return HIER_OK;
-  HIER_REQUIRE(a.items && a.kv_mask && a.out_items, HIER_EINVAL, "NULL pointer");
-  hipLaunchKernelGGL(trim_kernel, dim3(a.n_items), dim3(kTrimThreads), 0, (hipStream_t)stream, a);
-  return hier::check_launch("trim_kernel");
+  return trim_lists(*args, HierTrimArgs{}, stream);
+}
+
+extern "C" int hier_trim_key_lists2(const HierTrimArgs* a, const HierTrimArgs* b, void* stream) {
+  hier::clear_error();
+  HIER_REQUIRE(a != nullptr && b != nullptr, HIER_EINVAL, "args is NULL");
+  return trim_lists(*a, *b, stream);
 }

@@ -131,7 +131,8 @@ def hier_attention_backward(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, o
                             key_tiles: Optional[TileList] = None,
                             ste_geometry: Optional[tuple] = None,
                             ste_pass: str = "dq",
-                            no_alloc_workspace: bool = False):
+                            no_alloc_workspace: bool = False,
+                            ste_logits: Optional[torch.Tensor] = None):
     """``hier_attn_bwd``: gradients ``(dq, dk, dv)`` (bf16, shaped like q/k/v) of
     ``hier_attention_forward(q, k, v, tiles)`` given its output, its ``lse``
     and the output gradient.  ``tiles`` must be a full-sequence tile list;
@@ -142,7 +143,9 @@ def hier_attention_backward(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, o
     as an fp32 ``[T, N, P]`` tensor (see ``membership_grad``).  The sums are
     taken inside the dQ pass over the forward list's gated entries
     (``ste_pass="dq"``, the default) or by a separate pass over the STE list
-    (``ste_pass="list"``); both give the same sums up to fp32 rounding.
+    (``ste_pass="list"``); both give the same sums up to fp32 rounding.  With
+    ``ste_logits`` (fp32 ``[T, N, P]``, contiguous) the fourth result is their
+    gradient, ``membership_grad(ste_logits, sums)``, from the same launch.
 
     ``no_alloc_workspace=True`` calls ``hier_attn_bwd_noalloc``, whose
     per-row workspace lives in the library's device array instead of a
@@ -252,7 +255,13 @@ def hier_attention_backward(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, o
     red = _capi.HierSteReduceArgs(H=H, P=P_, T=T_, L=L_, N=N_, KL=KL_, classes=n_cls,
                                   partial=partial.data_ptr(), stride_h=partial.stride(0),
                                   out=sums.data_ptr())
-    _capi.call("hier_ste_reduce", C.byref(red), _stream(dev))
+    if ste_logits is None:
+        _capi.call("hier_ste_reduce", C.byref(red), _stream(dev))
+    else:
+        if ste_logits.shape != sums.shape or ste_logits.dtype != torch.float32 or \
+                ste_logits.device != sums.device or not ste_logits.is_contiguous():
+            raise ValueError("ste_logits must be contiguous fp32 [T, N, P] on q's device")
+        _capi.call("hier_ste_logit_grad", C.byref(red), ste_logits.data_ptr(), _stream(dev))
     return res + (sums,)
 
 
@@ -311,10 +320,17 @@ class HierAttentionFunction(torch.autograd.Function):
         q, k, v, out, lse = saved[:5]
         logits = saved[5] if len(saved) > 5 else None
         want_ste = logits is not None and ctx.needs_input_grad[5]
+        # (logits on another device, shaped with leading ones, or a backward
+        # that is itself recorded: by membership_grad)
+        direct = want_ste and logits.device == q.device and not torch.is_grad_enabled() and \
+            tuple(logits.shape) == tuple(ctx.ste_geometry[i] for i in (1, 3, 0))
         res = hier_attention_backward(q, k, v, out, dout.contiguous().to(torch.bfloat16), lse,
                                       ctx.tiles, scale=ctx.scale,
-                                      ste_geometry=ctx.ste_geometry if want_ste else None)
-        dlogits = membership_grad(logits, res[3]) if want_ste else None
+                                      ste_geometry=ctx.ste_geometry if want_ste else None,
+                                      ste_logits=logits.float().contiguous() if direct else None)
+        dlogits = None
+        if want_ste:
+            dlogits = res[3].to(logits.dtype) if direct else membership_grad(logits, res[3])
         return res[0], res[1], res[2], None, None, dlogits, None
 
 

@@ -651,7 +651,13 @@ class _HubMerge:
     def run(self, items, kv_idx, kv_mask, blk_and, n_items: int, stream):
         """Merged lists into their slots; the shared list's items and the
         forward list's items (None without folded rows)."""
-        out = torch.empty((max(self.n_out_items, 1), 8), dtype=torch.int32, device=items.device)
+        # with merged hub items only (none folded), they take the place of the
+        # hub items they replace, in front of the players' (the scatter, which
+        # reads those, has run by then): the shared list is a slice
+        at = self.first_player - self.n_items
+        in_place = self.merge and self.fwd_index is None and at >= 0
+        out = items[at:] if in_place else \
+            torch.empty((max(self.n_out_items, 1), 8), dtype=torch.int32, device=items.device)
         d = self._dev
         a = _capi.HierMergeArgs(
             n_groups=self.n_all_groups, n_src=self.n_src, rows=self.rows, rows_per_item=self.rpi,
@@ -659,6 +665,8 @@ class _HubMerge:
             blk_and=blk_and.data_ptr(), acc=self.acc.data_ptr(),
             **{k: v.data_ptr() for k, v in d.items()}, out_items=out.data_ptr())
         _capi.call("hier_merge_hub_lists", C.byref(a), stream)
+        if in_place:
+            return items[at:n_items], None
         kept = items[self.first_player:n_items]
         shared = torch.cat([out[:self.n_items], kept]) if self.merge else items[:n_items]
         if self.fwd_index is None:
@@ -1318,6 +1326,24 @@ def launch_list(tiles: TileList) -> TileList:
     fwd = None
     if tiles.fwd_items is not None:
         fwd = _trim_items(tiles.fwd_items, tiles.fwd_n_items, tiles.kv_mask, tiles.row_table)
+    return _set_launch(tiles, items, fwd)
+
+
+def _launch_pair(a: TileList, b: TileList) -> None:
+    """``launch_list`` of two new device lists without folded rows, in one
+    launch."""
+    outs = [torch.empty_like(t.items) for t in (a, b)]
+    args = [_capi.HierTrimArgs(n_items=t.n_items, items=t.items.data_ptr(),
+                               kv_mask=t.kv_mask.data_ptr(), row_table=None, out_items=o.data_ptr())
+            for t, o in zip((a, b), outs)]
+    _capi.call("hier_trim_key_lists2", C.byref(args[0]), C.byref(args[1]),
+               _capi.stream_of(a.items.device))
+    for t, o in zip((a, b), outs):
+        _set_launch(t, o, None)
+
+
+def _set_launch(tiles: TileList, items: torch.Tensor, fwd: Optional[torch.Tensor]) -> TileList:
+    """Keeps the cut items as ``tiles``'s launch list."""
     run = dataclasses.replace(tiles, items=items, fwd_items=fwd)
     # no reference back to a strong owner: a list built every training step
     # is freed when its last user drops it, without the cycle collector
@@ -1618,8 +1644,7 @@ class MembershipLogitsPlan:
                       merged_blocks=sup.merged_blocks)
         tiles.__dict__["_derived"] = {None: (kt, None)}
         tiles._keepalive = (self, a, lg)
-        launch_list(tiles)
-        launch_list(kt)
+        _launch_pair(tiles, kt)
         return tiles
 
 

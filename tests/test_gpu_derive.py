@@ -192,3 +192,52 @@ def test_logits_plan_equals_host_topology(case):
         torch.cuda.synchronize()
         for name, a, b in zip(("out", "dq", "dk", "dv", "dlogits"), *res):
             assert torch.equal(a, b), (seed, name)
+
+
+@pytest.mark.parametrize("P,T,N,L,KL", [(1, 1, 1, 1, 1), (4, 6, 2, 9, 3), (16, 3, 5, 300, 2),
+                                        (3, 4, 16, 1, 0)])
+def test_logit_gradient_from_the_reduction(P, T, N, L, KL):
+    """``hier_ste_logit_grad`` equals sigmoid' times ``hier_ste_reduce`` (the
+    same sums: one fp32 product and an exp apart), logits far from 0 included."""
+    need_gpu()
+    from multics_amd import _capi
+    say("logit gradient", P, T, N, L, KL)
+    H, ncls = 3, max(P, N)
+    g = torch.Generator(device="cuda").manual_seed(P + T)
+    part = torch.randn(H, P * T * L + T * N * KL, ncls, generator=g, device="cuda")
+    lg = 8 * torch.randn(T, N, P, generator=g, device="cuda")
+    lg.view(-1)[0] = 200.0
+    outs = [torch.full((T, N, P), float("nan"), device="cuda") for _ in range(2)]
+    for out, name, extra in ((outs[0], "hier_ste_reduce", ()),
+                             (outs[1], "hier_ste_logit_grad", (lg.data_ptr(),))):
+        a = _capi.HierSteReduceArgs(H=H, P=P, T=T, L=L, N=N, KL=KL, classes=ncls,
+                                    partial=part.data_ptr(), stride_h=part.stride(0),
+                                    out=out.data_ptr())
+        _capi.call(name, M.C.byref(a), *extra, _capi.stream_of(part.device))
+    torch.cuda.synchronize()
+    sig = torch.sigmoid(lg.double())
+    want = sig * (1 - sig) * outs[0].double()
+    # 1 - sigmoid carries the rounding of sigmoid: 2^-24 absolute on the factor
+    assert ((outs[1].double() - want).abs() <= 2e-7 * outs[0].double().abs() + 1e-6 * want.abs()).all()
+
+
+def test_two_lists_cut_in_one_launch():
+    """``hier_trim_key_lists2`` equals ``hier_trim_key_lists`` on each list, an
+    empty one on either side included."""
+    need_gpu()
+    from multics_amd import _capi
+    topo, tiles, _, _ = bench.build_case("c5", torch.device("cuda", 0))
+    kt = M.transpose_tiles(tiles)
+    say("two lists in one launch")
+    stream = _capi.stream_of(tiles.items.device)
+    for n_a, n_b in ((tiles.n_items, kt.n_items), (0, kt.n_items), (tiles.n_items, 0), (0, 0)):
+        outs = [torch.full_like(t.items, -7) for t in (tiles, kt)]
+        args = [_capi.HierTrimArgs(n_items=n, items=t.items.data_ptr(),
+                                   kv_mask=t.kv_mask.data_ptr(), row_table=None,
+                                   out_items=o.data_ptr())
+                for t, n, o in ((tiles, n_a, outs[0]), (kt, n_b, outs[1]))]
+        _capi.call("hier_trim_key_lists2", M.C.byref(args[0]), M.C.byref(args[1]), stream)
+        torch.cuda.synchronize()
+        for t, n, o in ((tiles, n_a, outs[0]), (kt, n_b, outs[1])):
+            assert torch.equal(o[:n], M._trim_items(t.items, t.n_items, t.kv_mask, None)[:n])
+            assert (o[n:] == -7).all()
