@@ -412,26 +412,34 @@ __global__ __launch_bounds__(kThreads) void meta_build_kernel(HierTopo t, HierMe
 
   // ---- attention tile list --------------------------------------------------
   if (out.tile_kv_idx) {
-    for (int r = threadIdx.x; r < R; r += kThreads) sh.val[r] = sh.mask[r] ? sh.width[r] : 0;
+    // a live run's first token, once per run (doff is free here): decoding it
+    // for every entry was a chain of frame-table loads per key
+    for (int r = threadIdx.x; r < R; r += kThreads) {
+      const bool live = sh.mask[r] != 0;
+      sh.val[r] = live ? sh.width[r] : 0;
+      sh.doff[r] = live ? tile_base(c, decode(c, kind, s, r)) : 0;
+    }
     __syncthreads();
     int uni = lds_excl_prefix(sh.val, sh.off, R, sh.tmp4);
     int padded = (uni + kTileKeys - 1) / kTileKeys * kTileKeys;
     int64_t base = out.tile_kv_off[(int64_t)c.b * NS + s];
-    int pad_idx = 0;
-    if (uni > 0) {
-      int r0 = find_run(sh.off, R, 0);
-      pad_idx = tile_base(c, decode(c, kind, s, r0));
-    }
-    for (int i = threadIdx.x; i < padded; i += kThreads) {
-      int idx = pad_idx;
-      uint32_t m = 0;
-      if (i < uni) {
-        int r = find_run(sh.off, R, i);
-        idx = tile_base(c, decode(c, kind, s, r)) + (i - sh.off[r]);
-        m = sh.mask[r];
+    const int pad_idx = uni > 0 ? sh.doff[find_run(sh.off, R, 0)] : 0;
+    // four consecutive entries per thread: one search, then steps to the next run
+    for (int i0 = 4 * threadIdx.x; i0 < padded; i0 += 4 * kThreads) {
+      int r = i0 < uni ? find_run(sh.off, R, i0) : 0;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int i = i0 + e;
+        int idx = pad_idx;
+        uint32_t m = 0;
+        if (i < uni) {
+          while (r + 1 < R && sh.off[r + 1] <= i) ++r;
+          idx = sh.doff[r] + (i - sh.off[r]);
+          m = sh.mask[r];
+        }
+        out.tile_kv_idx[base + i] = idx;
+        out.tile_kv_mask[base + i] = m;
       }
-      out.tile_kv_idx[base + i] = idx;
-      out.tile_kv_mask[base + i] = m;
     }
     for (int k = threadIdx.x; k < padded / kTileKeys; k += kThreads) {
       uint32_t a = ~0u;
@@ -660,12 +668,18 @@ extern "C" int hier_meta_build(const HierTopo* topo, const HierMetaOut* out, voi
 // lists cut in one launch (hier_trim_key_lists2) and the logits' gradient in
 // the STE reduction's (hier_ste_logit_grad), a training step of 4 players, 9
 // frames of 40 tokens, 8 heads went from 219 to 170 us, one of 8 players, 18
-// frames of 60, 12 heads from 812 to 774 us.
+// frames of 60, 12 heads from 812 to 774 us.  Inside a pass the time is a
+// chain of dependent loads and barriers, not bytes: what an entry needs is
+// looked up once per run or unit and kept in LDS, scans are by shuffles, a
+// list is one workgroup of 1024.  At 4 players, 21 frames of 220 tokens: lists
+// of the tile builder 29.7 -> 19.2 us, key-major lists 18.9 -> 11.2, entry
+// classes 19.0 -> 8.9, merged hub lists 16.7 -> 16.0.
 
 namespace {
 
 constexpr int kDeriveThreads = 256;
 constexpr int kScanThreads = 1024;
+constexpr int kClassThreads = 1024;     // one list per workgroup, ~100 workgroups: wide ones
 constexpr int kClasses = 64;            // STE classes (players or groups, <= 62)
 constexpr int64_t kMaxTable = 1ll << 26;  // n_groups^2 * nq_max table entries
 constexpr int kRunSplit = 8;            // workgroups per group list in the runs pass
@@ -733,21 +747,26 @@ __global__ void derive_fill_kernel(int32_t* p, int64_t n, int32_t v) {
     p[i] = v;
 }
 
-// Block-wide exclusive scan of one value per thread (kScanThreads threads).
+// Block-wide exclusive scan of one value per thread (kScanThreads threads):
+// the waves by shuffles, then the wave totals.
 __device__ int64_t block_scan(int64_t v, int64_t* sh, int64_t* total) {
-  const int t = threadIdx.x;
-  sh[t] = v;
-  __syncthreads();
-  for (int d = 1; d < kScanThreads; d <<= 1) {
-    const int64_t x = t >= d ? sh[t - d] : 0;
-    __syncthreads();
-    sh[t] += x;
-    __syncthreads();
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  int64_t incl = v;
+  for (int d = 1; d < 64; d <<= 1) {
+    const int64_t y = __shfl_up(incl, d);
+    if (lane >= d) incl += y;
   }
-  const int64_t incl = sh[t];
-  *total = sh[kScanThreads - 1];
+  __syncthreads();   // sh may still be read by a scan before this one
+  if (lane == 63) sh[wave] = incl;
   __syncthreads();
-  return incl - v;
+  int64_t before = 0, sum = 0;
+  for (int w = 0; w < kScanThreads / 64; ++w) {
+    const int64_t x = sh[w];
+    before += w < wave ? x : 0;
+    sum += x;
+  }
+  *total = sum;
+  return before + incl - v;
 }
 
 // First launch of pass 1.  blockIdx.y = 0 .. 2: tok_g cleared to -1, table and
@@ -756,7 +775,7 @@ __device__ int64_t block_scan(int64_t v, int64_t* sh, int64_t* total) {
 // (Independent work in one launch: each of these passes is a few
 // microseconds of latency.)
 __global__ __launch_bounds__(kScanThreads) void derive_init_kernel(HierDeriveArgs a, DeriveWs w) {
-  __shared__ int64_t sh[kScanThreads];
+  __shared__ int64_t sh[kScanThreads / 64];
   const int t = threadIdx.x;
   if (blockIdx.y < 3) {
     const int64_t tab = (int64_t)a.n_groups * a.n_groups * a.nq_max;
@@ -925,17 +944,18 @@ __global__ __launch_bounds__(kDeriveThreads) void derive_key_sizes_kernel(HierDe
 }
 
 // STE selection of one entry (key k, mask m) of the list of the group whose
-// query rows start at token qbase: class, or -1 if not kept.
+// query rows start at token qbase: class, or -1 if not kept.  (32-bit divisions:
+// k is one of the operands, and 64-bit ones are tens of instructions.)
 __device__ __forceinline__ int ste_class_at(const HierDeriveArgs& a, int64_t qbase, int k,
                                             uint32_t m) {
   const int64_t a0 = (int64_t)a.P * a.T * a.L, g0 = a0 + (int64_t)a.T * a.N * a.KL;
   if (m == 0 || k < 0 || qbase >= g0) return -1;
   if (qbase < a0) {
     if (k < a0 || k >= g0) return -1;
-    return (int)(((k - a0) / max(a.KL, 1)) % max(a.N, 1));
+    return (int)((uint32_t)(k - (int)a0) / (uint32_t)max(a.KL, 1) % (uint32_t)max(a.N, 1));
   }
   if (k >= a0) return -1;
-  return (int)(k / ((int64_t)a.T * a.L));
+  return (int)((uint32_t)k / (uint32_t)min((int64_t)a.T * a.L, (int64_t)UINT32_MAX));
 }
 
 __device__ __forceinline__ int ste_class(const HierDeriveArgs& a, const GroupDesc& d, int k,
@@ -947,9 +967,9 @@ __device__ __forceinline__ int ste_class(const HierDeriveArgs& a, const GroupDes
 // range (the items of a group write the same values; a cut item covers part
 // of its group's list; entries outside [0, kv_len) are never written), and
 // the first 64-entry tile of the item's range holding a class.
-__global__ __launch_bounds__(kDeriveThreads) void derive_fwd_class_kernel(HierDeriveArgs a,
-                                                                         int32_t* cls,
-                                                                         int32_t* first) {
+__global__ __launch_bounds__(kClassThreads) void derive_fwd_class_kernel(HierDeriveArgs a,
+                                                                        int32_t* cls,
+                                                                        int32_t* first) {
   __shared__ int s_first;
   const int32_t* it = a.items + 8 * (int64_t)blockIdx.x;
   const int64_t qbase = it[0], off = it[5], cnt = it[6];
@@ -997,7 +1017,7 @@ __global__ __launch_bounds__(kDeriveThreads) void derive_ste_count_kernel(HierDe
 
 // Offsets of the STE lists and items; totals [2] STE entries, [3] STE items.
 __global__ __launch_bounds__(kScanThreads) void derive_scan_kernel(HierDeriveArgs a, DeriveWs w) {
-  __shared__ int64_t sh[kScanThreads];
+  __shared__ int64_t sh[kScanThreads / 64];
   int64_t cs = 0, ci = 0;
   for (int base = 0; base < a.n_groups; base += kScanThreads) {
     const int g = base + threadIdx.x;
@@ -1031,9 +1051,10 @@ __global__ __launch_bounds__(kScanThreads) void derive_scan_kernel(HierDeriveArg
 // the caller's size: the backward then reads nothing through them).
 __global__ __launch_bounds__(kScanThreads) void derive_key_write_kernel(HierDeriveArgs a,
                                                                         DeriveWs w) {
-  __shared__ int64_t sh[kScanThreads];
-  __shared__ int32_t u_off[kScanThreads];
-  __shared__ int32_t u_id[kScanThreads];
+  __shared__ int64_t sh[kScanThreads / 64];
+  __shared__ int32_t u_off[kScanThreads];    // live units: first entry,
+  __shared__ int32_t u_row[kScanThreads];    // first query row,
+  __shared__ uint32_t u_mask[kScanThreads];  // frames of G it sees
   __shared__ int64_t base_s;
   const int G = blockIdx.x;
   const int ng = a.n_groups, nq = a.nq_max, nu = ng * nq;
@@ -1067,31 +1088,33 @@ __global__ __launch_bounds__(kScanThreads) void derive_key_write_kernel(HierDeri
   for (int u0 = 0; u0 < nu; u0 += kScanThreads) {
     const int u = u0 + threadIdx.x;
     const int g = u / nq;
-    const bool live = u < nu && row[u] != 0;
-    const int len = live ? group_desc(a, w, g).qlen : 0;
-    int64_t chunk, n_live;
-    const int64_t ex = block_scan(len, sh, &chunk);
-    // the live units of this chunk, compacted in order
-    const int64_t li = block_scan(live ? 1 : 0, sh, &n_live);
-    if (live) {
-      u_off[li] = (int32_t)ex;
-      u_id[li] = u;
+    const uint32_t sees = u < nu ? row[u] : 0u;
+    GroupDesc q{};
+    if (sees != 0) q = group_desc(a, w, g);
+    // entries before this unit, and live units before it (their order kept by
+    // the compaction) in the low bits: one scan for both
+    constexpr int kCountBits = 11;   // kScanThreads = 2^10 units
+    int64_t sums;
+    const int64_t ex = block_scan(sees != 0 ? ((int64_t)q.qlen << kCountBits) + 1 : 0, sh, &sums);
+    const int64_t chunk = sums >> kCountBits;
+    const int nl = (int)(sums & ((1 << kCountBits) - 1));
+    if (sees != 0) {
+      const int li = (int)(ex & ((1 << kCountBits) - 1));
+      u_off[li] = (int32_t)(ex >> kCountBits);
+      u_row[li] = q.qbase + (u - g * nq) * q.qstride;
+      u_mask[li] = sees;
     }
     __syncthreads();
-    const int nl = (int)n_live;
     for (int p = threadIdx.x; p < chunk; p += blockDim.x) {
       int lo = 0, hi = nl - 1;
       while (lo < hi) {
         const int mid = (lo + hi + 1) >> 1;
         if (u_off[mid] <= p) lo = mid; else hi = mid - 1;
       }
-      const int uu = u_id[lo], gg = uu / nq, j = uu - gg * nq;
-      const GroupDesc q = group_desc(a, w, gg);
-      const int r = p - u_off[lo];
       const int64_t o = base + done + p;
       if (o < lim) {
-        a.key_q_idx[o] = q.qbase + j * q.qstride + r;
-        a.key_q_mask[o] = row[uu];
+        a.key_q_idx[o] = u_row[lo] + (p - u_off[lo]);
+        a.key_q_mask[o] = u_mask[lo];
       }
     }
     done += chunk;
@@ -1102,11 +1125,14 @@ __global__ __launch_bounds__(kScanThreads) void derive_key_write_kernel(HierDeri
     a.key_q_mask[base + p] = 0;
   }
   __syncthreads();   // the masks are written
-  for (int t = threadIdx.x >> 6; t < padded / 64 && base + 64 * (int64_t)(t + 1) <= lim;
-       t += kScanThreads / 64) {   // one wave per tile
-    uint32_t v = a.key_q_mask[base + 64 * (int64_t)t + (threadIdx.x & 63)];
-    for (int d = 32; d >= 1; d >>= 1) v &= __shfl_xor(v, d);
-    if ((threadIdx.x & 63) == 0) a.key_blk_and[base / 64 + t] = v;
+  const int l16 = threadIdx.x & 15;   // 16 lanes per tile, four entries each
+  for (int t = threadIdx.x >> 4; t < padded / 64 && base + 64 * (int64_t)(t + 1) <= lim;
+       t += kScanThreads / 16) {
+    uint32_t v = ~0u;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) v &= a.key_q_mask[base + 64 * (int64_t)t + 16 * e + l16];
+    for (int d = 8; d >= 1; d >>= 1) v &= __shfl_xor(v, d, 16);
+    if (l16 == 0) a.key_blk_and[base / 64 + t] = v;
   }
 }
 
@@ -1274,7 +1300,7 @@ extern "C" int hier_derive_ste_classes(const HierDeriveArgs* args, int32_t* kv_c
   hipStream_t s = (hipStream_t)stream;
   fill(kv_class, a.kv_len, -1, s);
   if (a.n_items > 0)
-    hipLaunchKernelGGL(derive_fwd_class_kernel, dim3(a.n_items), dim3(kDeriveThreads), 0, s, a,
+    hipLaunchKernelGGL(derive_fwd_class_kernel, dim3(a.n_items), dim3(kClassThreads), 0, s, a,
                        kv_class, item_first);
   return hier::check_launch("derive_fwd_class_kernel");
 }
@@ -1429,12 +1455,22 @@ __global__ __launch_bounds__(kMergeThreads) void merge_compact_kernel(HierMergeA
   __syncthreads();
   // four consecutive rows per thread and pass, in row order: a thread's live
   // rows follow those of the lower lanes of its wave and of the lower waves
+  // (the next pass's masks are loaded before this pass's barriers)
   constexpr int kRows = 4 * kMergeThreads;
+  uint32_t next[4];
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    const int r = 4 * threadIdx.x + e;
+    next[e] = r < a.rows ? acc[r] : 0u;
+  }
   for (int r0 = 0; r0 < a.rows; r0 += kRows) {
     const int rb = r0 + 4 * threadIdx.x;
     uint32_t m[4];
 #pragma unroll
-    for (int e = 0; e < 4; ++e) m[e] = rb + e < a.rows ? acc[rb + e] : 0u;
+    for (int e = 0; e < 4; ++e) {
+      m[e] = next[e];
+      next[e] = (int64_t)rb + kRows + e < a.rows ? acc[rb + kRows + e] : 0u;
+    }
     const int mine = (m[0] != 0) + (m[1] != 0) + (m[2] != 0) + (m[3] != 0);
     int incl = mine;                       // inclusive prefix over the wave's lanes
 #pragma unroll
@@ -1472,10 +1508,13 @@ __global__ __launch_bounds__(kMergeThreads) void merge_compact_kernel(HierMergeA
     a.kv_mask[out + p] = 0;
   }
   __syncthreads();
-  for (int t = threadIdx.x; t < padded / 64; t += blockDim.x) {
+  // 16 lanes per tile, four entries each
+  for (int t = 4 * wave + (lane >> 4); t < padded / 64; t += 4 * (kMergeThreads / 64)) {
     uint32_t x = ~0u;
-    for (int e = 0; e < 64; ++e) x &= a.kv_mask[out + 64 * t + e];
-    a.blk_and[out / 64 + t] = x;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) x &= a.kv_mask[out + 64 * t + 16 * e + (lane & 15)];
+    for (int d = 8; d >= 1; d >>= 1) x &= __shfl_xor(x, d, 16);
+    if ((lane & 15) == 0) a.blk_and[out / 64 + t] = x;
   }
   // the group's items: rows split into rows_per_item pieces
   const int32_t* d = a.group_desc + 4 * (int64_t)g;      // qbase, qstride, qlen, frames

@@ -241,3 +241,19 @@ def test_two_lists_cut_in_one_launch():
         for t, n, o in ((tiles, n_a, outs[0]), (kt, n_b, outs[1])):
             assert torch.equal(o[:n], M._trim_items(t.items, t.n_items, t.kv_mask, None)[:n])
             assert (o[n:] == -7).all()
+
+
+@pytest.mark.parametrize("P,T,L", [(15, 63, 1), (16, 64, 3), (16, 130, 2)])
+def test_lists_of_many_groups(P, T, L):
+    """One query frame per block, so that the key-major builder walks its
+    (group, frame) units in one short chunk, about one full chunk of 1024 and
+    several: equal to the host's lists (short runs: entries of four share
+    several)."""
+    need_gpu()
+    dev = torch.device("cuda", 0)
+    say("many groups", P, T, L)
+    N, KL, KG, n, W = 1, 1, 1, 1, 4
+    tiles = M.full_sequence_tiles(device=dev, P=P, T=T, L=L, N=N, KL=KL, KG=KG, n=n, window=W,
+                                  direct=True, labels=np.zeros((T, P), int),
+                                  active=np.ones((T, N), bool))
+    _check_lists(tiles, (P, T, L, N, KL))
