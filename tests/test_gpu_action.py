@@ -45,7 +45,7 @@ def test_frame_attention_matches_oracle(D, local_attn):
 
 
 @pytest.mark.parametrize("D", [64, 128])
-@pytest.mark.parametrize("Lq", [1, 2, 3, 4, 5, 8, 9, 16, 17, 32, 33, 129])
+@pytest.mark.parametrize("Lq", [1, 2, 3, 4, 5, 6, 7, 8, 9, 14, 16, 17, 32, 33, 129])
 def test_frame_attention_edges(D, Lq):
     """Every kernel variant (waves of 1-8 queries, matrix tiles above) at
     the edges of its key chunks and tiles, with keys that no query, one query
