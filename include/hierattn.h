@@ -528,7 +528,8 @@ int hier_kv_append(const HierPageArgs* args, void* stream);
 /* blocks.py:374 (keyboard cross-attention), whose boolean mask is          */
 /*   visible(i, j) = k_frame[j] / n_block <= q_frame[i] / n_block           */
 /*                   and (local_attn == -1 or q_frame[i] - k_frame[j] < local_attn) */
-/* (blocks.py:303-306, 366-372).  Rows that see no key are written as 0.    */
+/* (blocks.py:303-306, 366-372).  Rows that see no key are written as 0; a  */
+/* key that a query does not see adds nothing to its row, whatever it holds. */
 /* Element (b, s, h, d) of q / k / v / o is at b*_sb + s*_ss + h*_sh + d.   */
 /* ------------------------------------------------------------------------ */
 typedef struct HierFrameAttnArgs {

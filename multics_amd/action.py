@@ -49,7 +49,7 @@ def frame_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, q_frame: 
     key j is visible to query i when ``k_frame[j] // n_block <= q_frame[i] //
     n_block`` and, for ``local_attn != -1``, ``q_frame[i] - k_frame[j] <
     local_attn``.  Returns ``[B, Lq, H, D]`` bf16 (0 for a query that sees
-    no key)."""
+    no key; rows that a query does not see may hold infinities or NaN)."""
     if torch.is_grad_enabled() and any(t.requires_grad for t in (q, k, v)):
         raise RuntimeError("frame-window attention is inference-only (q/k/v require grad); run "
                            "the cached action branches under torch.no_grad() or "

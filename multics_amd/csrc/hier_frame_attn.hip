@@ -22,6 +22,13 @@
 //               loaded during the current one.  Bound by the latency of its
 //               few steps.  10 x 24 heads, 660 x 96 keys: 34 us (329 us with
 //               one key at a time per query).
+//
+// Both give every key a weight, 0 where the mask hides it, and 0 times an
+// infinity or a NaN is a NaN.  A hidden row counts for nothing whatever it
+// holds, so where results are not all finite, or a query's weights sum to 0,
+// a wave computes its queries again from their visible keys alone, a key at a
+// time (visible_only).  The check costs the keyboard branch 2 us of 38, waves
+// of 7 or 8 queries 1-3 %, the temporal branch nothing.
 #include "hier_common.h"
 #include "hier_launch.h"
 #include "hier_tile.h"
@@ -70,6 +77,77 @@ __device__ __forceinline__ float fold16(float a, float b) {   // rows 0, 2: a's 
 __device__ __forceinline__ float max16(float v) {
   const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
   return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
+}
+
+// Sum of packed results: infinite or NaN if one of them is.
+__device__ __forceinline__ float probe(uint32_t w, float sum) {
+  return __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2, w),
+                                         __builtin_bit_cast(bf16x2, 0x3f803f80u), sum, false);
+}
+// A weight sum of 0, or it or a sum of results infinite or NaN.  (By their bits and out
+// of the compiler's sight: this is built to assume that no NaN occurs.)
+__device__ __forceinline__ bool is_odd(float l, float sum) {
+  uint32_t w = __float_as_uint(l), x = __float_as_uint(sum);
+  asm("" : "+v"(w), "+v"(x));
+  return w - 1u >= 0x7f7fffffu || (x & 0x7f800000u) == 0x7f800000u;
+}
+
+// Queries [q0, q0 + nq) of a (sequence, head) by one wave, from the keys that
+// each sees and no others: D / 8 lanes per query, a key at a time, the running
+// maximum from -infinity.
+template <int D>
+__device__ __forceinline__ void visible_only(const HierFrameAttnArgs& a, int64_t b, int64_t h,
+                                             int q0, int nq) {
+  // (a score is rounded before the maximum is taken off: fused, what that
+  // leaves of -1e31 is not 0)
+#pragma clang fp contract(off)
+  constexpr int LPR = D / 8, R = 64 / LPR;
+  const int lane = threadIdx.x & 63, c = lane % LPR, r = lane / LPR;
+  const uint16_t* const kb = a.k + b * a.k_sb + h * a.k_sh + 8 * c;
+  const uint16_t* const vb = a.v + b * a.v_sb + h * a.v_sh + 8 * c;
+  const float c2 = a.scale * kLog2e;
+#pragma unroll 1
+  for (int i = r; i - r < nq; i += R) {
+    const bool mine = i < nq && q0 + i < a.Lq;
+    const int qi = min(q0 + i, a.Lq - 1);
+    const u32x4 q = *reinterpret_cast<const u32x4*>(a.q + b * a.q_sb + (int64_t)qi * a.q_ss +
+                                                    h * a.q_sh + 8 * c);
+    Window win;
+    win.init(a.q_frame[qi], a.n_block, a.local_attn);
+    float m = -INFINITY, l = 0.f, o[8] = {};
+#pragma unroll 1
+    for (int j = 0; j < a.Lk; ++j) {
+      const u32x4 k = *reinterpret_cast<const u32x4*>(kb + (int64_t)j * a.k_ss);
+      const u32x4 v = *reinterpret_cast<const u32x4*>(vb + (int64_t)j * a.v_ss);
+      float s = 0.f;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const uint32_t x = q[e], y = k[e];
+        s = __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2, x),
+                                            __builtin_bit_cast(bf16x2, y), s, false);
+      }
+#pragma unroll
+      for (int d = 1; d < LPR; d <<= 1) s += __shfl_xor(s, d, 64);
+      if (!win.sees(a.k_frame[j])) continue;
+      const float t = s * c2, mn = fmaxf(m, t);
+      const float alpha = __builtin_amdgcn_exp2f(m - mn);   // m = -inf: 0
+      const float p = __builtin_amdgcn_exp2f(t - mn);
+      l = fmaf(l, alpha, p);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        o[2 * e] = fmaf(p, lo(v[e]), o[2 * e] * alpha);
+        o[2 * e + 1] = fmaf(p, hi(v[e]), o[2 * e + 1] * alpha);
+      }
+      m = mn;
+    }
+    const float inv = l > 0.f ? 1.f / l : 0.f;
+    u32x4 w;
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      w[e] = (uint32_t)f2bf(o[2 * e] * inv) | ((uint32_t)f2bf(o[2 * e + 1] * inv) << 16);
+    if (mine)
+      *reinterpret_cast<u32x4*>(a.o + b * a.o_sb + (int64_t)qi * a.o_ss + h * a.o_sh + 8 * c) = w;
+  }
 }
 
 // ---- up to 8 queries per sequence ------------------------------------------
@@ -215,6 +293,7 @@ __global__ __launch_bounds__(256, LOOP || NQ > 4 ? 2 : 3) void seq_kernel(HierFr
   // Sums over the row groups, four queries at a time: lane row 0 / 1 / 2 / 3
   // (16 lanes) ends up with query 0 / 2 / 1 / 3 of the four, and stores it.
   const int rw = lane >> 4, qr = (rw & 1) << 1 | rw >> 1;
+  bool odd[(NQ + 3) / 4];
 #pragma unroll
   for (int i0 = 0; i0 < NQ; i0 += 4) {
     auto fold = [&](auto get) {
@@ -229,16 +308,23 @@ __global__ __launch_bounds__(256, LOOP || NQ > 4 ? 2 : 3) void seq_kernel(HierFr
     const float lt = fold([&](int i) { return l[i]; });
     const float inv = lt > 0.f ? 1.f / lt : 0.f;
     u32x4 w;
+    float sum = 0.f;
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
       const float x = fold([&](int i) { return o[i][2 * e]; }) * inv;
       const float y = fold([&](int i) { return o[i][2 * e + 1]; }) * inv;
       w[e] = (uint32_t)f2bf(x) | ((uint32_t)f2bf(y) << 16);
+      sum = probe(w[e], sum);
     }
-    if (i0 + qr < NQ && q0 + i0 + qr < a.Lq && (LPR == 16 || (lane & 8) == 0))
+    const bool mine = i0 + qr < NQ && q0 + i0 + qr < a.Lq;
+    odd[i0 / 4] = __ballot(mine && is_odd(lt, sum)) != 0;
+    if (!odd[i0 / 4] && mine && (LPR == 16 || (lane & 8) == 0))
       *reinterpret_cast<u32x4*>(a.o + (int64_t)b * a.o_sb + (int64_t)(q0 + i0 + qr) * a.o_ss +
                                 (int64_t)h * a.o_sh + 8 * c) = w;
   }
+  if (odd[0]) visible_only<D>(a, b, h, q0, min(NQ, 4));
+  if constexpr (NQ > 4)
+    if (odd[1]) visible_only<D>(a, b, h, q0 + 4, NQ - 4);
 }
 
 // ---- more queries: matrix-core tiles ----------------------------------------
@@ -363,19 +449,34 @@ __global__ __launch_bounds__(256, 2) void tile_kernel(HierFrameAttnArgs a, int q
         }
     }
   }
-  if (q0 + (lane & 31) >= a.Lq) return;
+  if (!active) return;
   const float lt = pair_sum(l);
   const float inv = lt > 0.f ? 1.f / lt : 0.f;
+  u32x2 res[NDB][4];
+  float sum = 0.f;
+#pragma unroll
+  for (int i = 0; i < NDB; ++i)
+#pragma unroll
+    for (int g4 = 0; g4 < 4; ++g4)
+#pragma unroll
+      for (int e = 0; e < 2; ++e) {
+        const uint32_t w = (uint32_t)f2bf(o[i][4 * g4 + 2 * e] * inv) |
+                           ((uint32_t)f2bf(o[i][4 * g4 + 2 * e + 1] * inv) << 16);
+        res[i][g4][e] = w;
+        sum = probe(w, sum);
+      }
+  const bool stored = q0 + (lane & 31) < a.Lq;
+  if (__ballot(stored && is_odd(lt, sum)) != 0) {
+    visible_only<D>(a, b, h, q0, 32);
+    return;
+  }
+  if (!stored) return;
   uint16_t* op = a.o + (int64_t)b * a.o_sb + (int64_t)qi * a.o_ss + (int64_t)h * a.o_sh;
 #pragma unroll
   for (int i = 0; i < NDB; ++i)
 #pragma unroll
-    for (int g4 = 0; g4 < 4; ++g4) {
-      u32x2 w;
-      w[0] = (uint32_t)f2bf(o[i][4 * g4] * inv) | ((uint32_t)f2bf(o[i][4 * g4 + 1] * inv) << 16);
-      w[1] = (uint32_t)f2bf(o[i][4 * g4 + 2] * inv) | ((uint32_t)f2bf(o[i][4 * g4 + 3] * inv) << 16);
-      *reinterpret_cast<u32x2*>(op + i * 32 + 8 * g4 + 4 * (lane >> 5)) = w;
-    }
+    for (int g4 = 0; g4 < 4; ++g4)
+      *reinterpret_cast<u32x2*>(op + i * 32 + 8 * g4 + 4 * (lane >> 5)) = res[i][g4];
 }
 
 // Queries that one wave of seq_kernel holds: 8 of a window of one chunk (32 or

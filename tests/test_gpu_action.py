@@ -82,6 +82,67 @@ def test_frame_attention_edges(D, Lq):
         assert (got.cpu()[:, ~m.any(1)] == 0).all()
 
 
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("Lq,Lk", [(3, 24), (7, 40), (12, 70), (3, 200), (40, 96)])
+def test_frame_attention_hidden_rows_count_for_nothing(D, Lq, Lk):
+    """A key outside a query's window leaves that query's result alone whatever
+    its K and V rows hold (infinities, NaN), in every kernel: the last row
+    among them, which stands in for the rows past it, and rows that other
+    queries see (whose results are then as without a mask: an infinity where V
+    is infinite, NaN where a NaN takes part).  A query that sees nothing gives
+    0.  Bounds as in test_frame_attention_edges."""
+    need_gpu()
+    say("frame attention hidden rows", D, Lq, Lk)
+    g = torch.Generator().manual_seed(Lq + Lk + D)
+    B, H, W = 2, 3, 6
+    q, k, v = (torch.randn(B, L, H, D, generator=g).to(torch.bfloat16) for L in (Lq, Lk, Lk))
+    kf = 20 + torch.arange(Lk) * 20 // Lk
+    qf = torch.linspace(28, 36, Lq).long()           # frames 20-39: hidden on both sides
+    qf[0] = 5                                        # sees nothing
+    vis = (kf[None] <= qf[:, None]) & (qf[:, None] - kf[None] < W)
+    hidden = ~vis.any(0)
+    assert hidden[-1] and hidden[0]
+    bad = torch.zeros(Lk, dtype=torch.bool)
+    bad[-1] = bad[0] = True
+    for rows, value in ((bad, float("nan")), (bad, float("inf")), (hidden, float("-inf"))):
+        kk, vv = k.clone(), v.clone()
+        kk[:, rows], vv[:, rows] = value, value
+        # a row that only the queries of its own window see
+        one = int((kf == 30).nonzero()[0])
+        vv[:, one, :, 1] = float("inf")
+        vv[:, one, :, 2] = float("nan")
+        got = frame_attention(q.cuda(), kk.cuda(), vv.cuda(), qf, kf, 1, W).double().cpu()
+        torch.cuda.synchronize()
+        sc = torch.einsum("bihd,bjhd->bhij", q.double(), k.double()) / math.sqrt(D)
+        p = torch.softmax(sc.masked_fill(~vis, -math.inf), -1).nan_to_num(0.0)
+        ref = torch.einsum("bhij,bjhd->bihd", p, v.double())
+        sees = vis[:, one]
+        ref[:, sees, :, 1], ref[:, sees, :, 2] = math.inf, math.nan
+        fin = torch.isfinite(ref)
+        err = (got[fin] - ref[fin]).abs()
+        assert (err <= 2.0 ** -8 * ref[fin].abs() + 1e-3).all(), float(err.max())
+        assert (got[:, sees, :, 1] == math.inf).all() and got[:, sees, :, 2].isnan().all()
+        assert (got[:, 0] == 0).all()
+
+
+@pytest.mark.parametrize("Lq,Lk", [(3, 24), (3, 200), (40, 96)])
+def test_frame_attention_scores_far_below_zero(Lq, Lk):
+    """Scores of any finite size weigh their keys: one of -1e31 beside others
+    that are lower by far takes the whole weight."""
+    need_gpu()
+    say("frame attention low scores", Lq, Lk)
+    D = 128
+    g = torch.Generator().manual_seed(Lk)
+    q = torch.full((1, Lq, 2, D), 1e15).to(torch.bfloat16)
+    k = torch.full((1, Lk, 2, D), -2e16).to(torch.bfloat16)
+    k[:, Lk // 2] = -1e15
+    v = torch.randn(1, Lk, 2, D, generator=g).to(torch.bfloat16)
+    got = frame_attention(q.cuda(), k.cuda(), v.cuda(), torch.full((Lq,), 9),
+                          torch.arange(Lk) % 10, 10, -1).cpu()
+    torch.cuda.synchronize()
+    assert torch.equal(got, v[:, Lk // 2:Lk // 2 + 1].expand_as(got))
+
+
 class _Attn(nn.Module):
     """The attributes the reference's cached action attention reads."""
 
