@@ -3,7 +3,7 @@
 // keyboard cross-attention over a rolling cache).  Key j is visible to query i
 // when k_frame[j] / n_block <= q_frame[i] / n_block and, with a window,
 // q_frame[i] - k_frame[j] < local_attn.  Scores, softmax weights and sums are
-// fp32 (the weights multiply V as two bf16 parts where the matrix cores do it).
+// fp32 (the weights multiply V as three bf16 parts where the matrix cores do it).
 //
 // Two kernels, by the queries and keys of a sequence:
 //
@@ -20,14 +20,14 @@
 //               tokens per player): 128 queries per workgroup on the matrix
 //               cores, 64-key tiles of K and V in LDS, the next tile's rows
 //               loaded during the current one.  Bound by the latency of its
-//               few steps.  10 x 24 heads, 660 x 96 keys: 34 us (329 us with
+//               few steps.  10 x 24 heads, 660 x 96 keys: 39 us (329 us with
 //               one key at a time per query).
 //
 // Both give every key a weight, 0 where the mask hides it, and 0 times an
 // infinity or a NaN is a NaN.  A hidden row counts for nothing whatever it
 // holds, so where results are not all finite, or a query's weights sum to 0,
 // a wave computes its queries again from their visible keys alone, a key at a
-// time (visible_only).  The check costs the keyboard branch 2 us of 38, waves
+// time (visible_only).  The check costs the keyboard branch 2 us of 39, waves
 // of 7 or 8 queries 1-3 %, the temporal branch nothing.
 #include "hier_common.h"
 #include "hier_launch.h"
@@ -331,9 +331,10 @@ __global__ __launch_bounds__(256, LOOP || NQ > 4 ? 2 : 3) void seq_kernel(HierFr
 //
 // Four waves of 32 queries.  S^T = K Q^T leaves each lane one query and 16 keys
 // of a 32-key block (hier_tile.h); P goes from the accumulators into the
-// operand of O^T += V^T P^T as the bf16 of P and the bf16 of what that rounding
-// left (2^-17 of P together: the products with bf16 V are exact, the sums
-// fp32).  The rows reach LDS through registers: any row stride works.
+// operand of O^T += V^T P^T as the bf16 of P, the bf16 of what that rounding
+// left and the bf16 of what is left then: all 24 bits of P (the products with
+// bf16 V are exact, the sums fp32).  The rows reach LDS through registers: any
+// row stride works.
 
 template <int D>
 __global__ __launch_bounds__(256, 2) void tile_kernel(HierFrameAttnArgs a, int q_tiles, int total) {
@@ -429,14 +430,17 @@ __global__ __launch_bounds__(256, 2) void tile_kernel(HierFrameAttnArgs a, int q
           for (int e = 0; e < 16; ++e) o[i][e] *= alpha;
         m = mn;
       }
-      bf16x8 ph[2], pl[2];
+      bf16x8 ph[2], pm[2], pl[2];
 #pragma unroll
       for (int e = 0; e < 16; ++e) {
         const float p = __builtin_amdgcn_exp2f(s[e] - m);
         l += p;
         const __bf16 t = (__bf16)p;
         ph[e >> 3][e & 7] = t;
-        pl[e >> 3][e & 7] = (__bf16)(p - (float)t);
+        const float left = p - (float)t;         // exact, as the next
+        const __bf16 u = (__bf16)left;
+        pm[e >> 3][e & 7] = u;
+        pl[e >> 3][e & 7] = (__bf16)(left - (float)u);
       }
 #pragma unroll
       for (int j = 0; j < 2; ++j)
@@ -445,6 +449,7 @@ __global__ __launch_bounds__(256, 2) void tile_kernel(HierFrameAttnArgs a, int q
           const char* p0 = vt0 + j * 16 * ROWB + va[i];
           const bf16x8 vt = tr_read(p0, p0 + HALF);
           o[i] = mfma(vt, ph[j], o[i]);
+          o[i] = mfma(vt, pm[j], o[i]);
           o[i] = mfma(vt, pl[j], o[i]);
         }
     }

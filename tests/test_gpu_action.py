@@ -143,6 +143,34 @@ def test_frame_attention_scores_far_below_zero(Lq, Lk):
     assert torch.equal(got, v[:, Lk // 2:Lk // 2 + 1].expand_as(got))
 
 
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("Lq", [3, 40])
+def test_frame_attention_weights_are_fp32(D, Lq):
+    """Softmax weights multiply V with all their 24 bits in every kernel.  Keys
+    of weight 1, p and 1 carry v = hi, -1 and lo, the bf16 of p and the bf16
+    of what that leaves: the result is what two bf16 parts of p leave out,
+    over 2 + p.  Bound: the result's bf16 rounding (2^-9 of it) and the fp32
+    error of p (exp2 and score, 2^-23 together)."""
+    need_gpu()
+    say("frame attention weights", D, Lq)
+    H, scale = 48, 0.25
+    x = torch.linspace(0.3, 3.0, H).to(torch.bfloat16)
+    p = torch.exp(-x.double() * scale)
+    hi = p.to(torch.bfloat16)
+    lo = (p - hi.double()).to(torch.bfloat16)
+    q, k, v = (torch.zeros(1, L, H, D, dtype=torch.bfloat16) for L in (Lq, 3, 3))
+    q[..., 0] = 1
+    k[0, 1, :, 0] = -x
+    v[0, 0], v[0, 1], v[0, 2] = hi[:, None], -1, lo[:, None]
+    got = frame_attention(q.cuda(), k.cuda(), v.cuda(), torch.zeros(Lq), torch.zeros(3), 1, -1,
+                          scale=scale).double().cpu()
+    torch.cuda.synchronize()
+    ref = ((hi.double() - p + lo.double()) / (2 + p))[None, None, :, None].expand_as(got)
+    assert (ref.abs() > 2.0 ** -21).sum() > ref.numel() / 4   # seen above the bound
+    err = (got - ref).abs()
+    assert (err <= 2.0 ** -9 * ref.abs() + 2.0 ** -23).all(), float(err.max())
+
+
 class _Attn(nn.Module):
     """The attributes the reference's cached action attention reads."""
 
