@@ -32,35 +32,18 @@
 #include "hier_common.h"
 #include "hier_launch.h"
 #include "hier_tile.h"
-
-#include <climits>
+#include "hier_window.h"
 
 namespace {
 
 using namespace hier::tile;
+using hier::Window;
 
 constexpr float kLog2e = 1.4426950408889634f;
 constexpr float kNoMax = -1e30f;       // running max of a row without a visible key
 
 __device__ __forceinline__ float lo(uint32_t w) { return __uint_as_float(w << 16); }
 __device__ __forceinline__ float hi(uint32_t w) { return __uint_as_float(w & 0xffff0000u); }
-
-// The key frames that a query sees are an interval [first, first + span]: the
-// block rule bounds them above (n_block divides towards zero, as the host's
-// integer division of non-negative frames does), the window below.  It always
-// holds the query's own frame.
-struct Window {
-  int first;
-  uint32_t span;
-  __device__ __forceinline__ void init(int qf, int n_block, int local_attn) {
-    const int b = qf / n_block;
-    const int64_t last = (int64_t)b * n_block + (b >= 0 ? n_block - 1 : 0);
-    const int64_t f0 = local_attn < 0 ? (int64_t)INT_MIN : (int64_t)qf - local_attn + 1;
-    first = (int)max(f0, (int64_t)INT_MIN);
-    span = (uint32_t)(min(last, (int64_t)INT_MAX - 1) - first);   // INT_MAX marks no key
-  }
-  __device__ __forceinline__ bool sees(int kf) const { return (uint32_t)(kf - first) <= span; }
-};
 
 template <int CTRL>
 __device__ __forceinline__ float dpp(float v) {
