@@ -137,8 +137,8 @@ __device__ __forceinline__ void visible_only(const HierFrameAttnArgs& a, int64_t
 
 // One wave: NQ queries of a (sequence, head), the keys in one chunk of G row
 // groups or (LOOP) in several.  A sequence's ceil(Lq / NQ) waves sit side by side (in one
-// workgroup as a rule), so its rows come from memory once.
-template <int D, int NQ, int G, bool LOOP>
+// workgroup as a rule).  ONCE: that is one wave, and a row is read by it alone.
+template <int D, int NQ, int G, bool LOOP, bool ONCE>
 __global__ __launch_bounds__(256, LOOP || NQ > 4 ? 2 : 3) void seq_kernel(HierFrameAttnArgs a,
                                                                      uint32_t nqg, uint32_t units) {
   constexpr int LPR = D / 8;          // lanes per row
@@ -158,11 +158,14 @@ __global__ __launch_bounds__(256, LOOP || NQ > 4 ? 2 : 3) void seq_kernel(HierFr
   const uint16_t* const vr = vb + (int64_t)r * a.v_ss;
   u32x4 k[G], v[G];
   int kf[G];
-  // a row is read once, by one wave: past the caches (the temporal branch 132 us
-  // without, 115 with); in a loop the rows' neighbours follow (1,000 keys: 34 / 47)
+  // a row read once: past the caches.  24 keys x 24 heads of 128, 3 queries,
+  // plain / past them: 2,200 sequences 133 / 116 us, 400 27 / 25, 40 6.0 / 6.0.
+  // Two waves read the same rows: 2,200 sequences, 16 queries 309 / 321 us, 12
+  // queries 250 / 254, 40 sequences 9.5 / 10.4.  In a loop the rows' neighbours
+  // follow (1,000 keys: 34 / 47).
   auto load = [&](const uint16_t* p) {
     const u32x4* w = reinterpret_cast<const u32x4*>(p);
-    if constexpr (LOOP) return *w;
+    if constexpr (LOOP || !ONCE) return *w;
     else return __builtin_nontemporal_load(w);
   };
   auto fetch = [&](int j0) {          // a chunk's rows, all before any is used
@@ -471,43 +474,47 @@ __global__ __launch_bounds__(256, 2) void tile_kernel(HierFrameAttnArgs a, int q
 // 64 keys), 4 where it loops over chunks (each waits for its rows).
 bool one_chunk(const HierFrameAttnArgs& a) { return a.Lk <= 8 * (512 / a.D); }
 int query_groups(const HierFrameAttnArgs& a) { return one_chunk(a) ? (a.Lq + 7) / 8 : (a.Lq + 3) / 4; }
-// tile_kernel costs a sequence the same from 1 to 32 queries.  Windows of one
+// tile_kernel works on 32 queries whether they are there or not.  Windows of one
 // chunk (2,200 x 24 heads, 24 keys, D = 128), seq_kernel / tile_kernel: 8
-// queries 181 / 415 us, 16 317 / 445, 32 623 / 499.  Longer (40 x 24 heads, 200
-// keys): 3 21 / 30 us, 5 28 / 30, 8 33 / 30; 8 heads, 1,000 keys: 5 59 / 37.
+// queries 173 / 445 us, 16 309 / 475, 24 472 / 508, 32 612 / 533; 40 x 24 heads:
+// 16 9.8 / 10.0, 24 13.4 / 10.4.  Longer (40 x 24 heads, 200 keys): 3 21 / 33 us,
+// 5 29 / 33, 8 33 / 34; 8 heads, 1,000 keys: 5 59 / 43.
 bool use_seq(const HierFrameAttnArgs& a) { return a.Lq <= (one_chunk(a) ? 16 : 4); }
 
-template <int D, int NQ>
+template <int D, int NQ, bool ONCE>
 void launch_seq(const HierFrameAttnArgs& a, hipStream_t st) {
   const int nqg = query_groups(a);
   const int64_t units = (int64_t)a.B * a.H * nqg;
   const dim3 grid((unsigned)((units + 3) / 4)), block(256);
   const int groups = (a.Lk + 512 / D - 1) / (512 / D);   // of 512 / D rows
 #define HIER_SEQ(G, LOOP) \
-  hipLaunchKernelGGL((seq_kernel<D, NQ, G, LOOP>), grid, block, 0, st, a, (uint32_t)nqg, (uint32_t)units)
+  hipLaunchKernelGGL((seq_kernel<D, NQ, G, LOOP, ONCE>), grid, block, 0, st, a, (uint32_t)nqg, (uint32_t)units)
   if (groups <= 2) HIER_SEQ(2, false);
   else if (groups <= 3) HIER_SEQ(3, false);
   else if (groups <= 4) HIER_SEQ(4, false);
   else if (groups <= 6) HIER_SEQ(6, false);
   else if (groups <= 8) HIER_SEQ(8, false);
-  else if constexpr (NQ <= 4) HIER_SEQ(8, true);
+  else if constexpr (ONCE && NQ <= 4) HIER_SEQ(8, true);
 #undef HIER_SEQ
 }
 
 template <int D>
 void launch_seq_d(const HierFrameAttnArgs& a, hipStream_t st) {
   const int nqg = query_groups(a);
+  // (up to 8 queries, or 4 in a loop, are one wave's; 9 to 16 are two waves' of 5 to 8)
+#define HIER_NQ(N) return nqg == 1 ? launch_seq<D, N, true>(a, st) : launch_seq<D, N, false>(a, st)
   switch ((a.Lq + nqg - 1) / nqg) {
-    case 1: return launch_seq<D, 1>(a, st);
-    case 2: return launch_seq<D, 2>(a, st);
-    case 3: return launch_seq<D, 3>(a, st);
-    case 4: return launch_seq<D, 4>(a, st);
+    case 1: return launch_seq<D, 1, true>(a, st);
+    case 2: return launch_seq<D, 2, true>(a, st);
+    case 3: return launch_seq<D, 3, true>(a, st);
+    case 4: return launch_seq<D, 4, true>(a, st);
     case 5:
-    case 6: return launch_seq<D, 6>(a, st);
+    case 6: HIER_NQ(6);
     // (7 as 8, 1,970 x 12 heads, 14 keys, D = 64: 50.9 us, as 7 46.9)
-    case 7: return launch_seq<D, 7>(a, st);
-    default: return launch_seq<D, 8>(a, st);
+    case 7: HIER_NQ(7);
+    default: HIER_NQ(8);
   }
+#undef HIER_NQ
 }
 
 }  // namespace
