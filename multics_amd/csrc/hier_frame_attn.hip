@@ -144,7 +144,7 @@ __global__ __launch_bounds__(256, LOOP || NQ > 4 ? 2 : 3) void seq_kernel(HierFr
   constexpr int LPR = D / 8;          // lanes per row
   constexpr int R = 64 / LPR;         // rows per group
   const int lane = threadIdx.x & 63;
-  const uint32_t unit = blockIdx.x * 4 + __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  const uint32_t unit = (blockIdx.y * gridDim.x + blockIdx.x) * 4 + __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
   if (unit >= units) return;
   const uint32_t bh = unit / nqg, b = bh / (uint32_t)a.H;
   const int h = (int)(bh - b * (uint32_t)a.H), q0 = (int)(unit - bh * nqg) * NQ;
@@ -330,7 +330,8 @@ __global__ __launch_bounds__(256, 2) void tile_kernel(HierFrameAttnArgs a, int q
   __shared__ __align__(16) int lds_f[kSlab];
   // the query tiles of one sequence and head on one XCD, which then reads
   // their keys from memory once
-  const int logical = hier::xcd_logical(blockIdx.x, gridDim.x);
+  const int logical = hier::xcd_logical((int)(blockIdx.y * gridDim.x + blockIdx.x),
+                                        (int)(gridDim.x * gridDim.y));
   if (logical >= total) return;
   const int bh = logical / q_tiles, b = bh / a.H, h = bh - b * a.H;
   const int tid = threadIdx.x, lane = tid & 63;
@@ -485,7 +486,8 @@ template <int D, int NQ, bool ONCE>
 void launch_seq(const HierFrameAttnArgs& a, hipStream_t st) {
   const int nqg = query_groups(a);
   const int64_t units = (int64_t)a.B * a.H * nqg;
-  const dim3 grid((unsigned)((units + 3) / 4)), block(256);
+  const hier::Grid gr = hier::launch_grid((units + 3) / 4, 256);
+  const dim3 grid(gr.x, gr.y), block(256);
   const int groups = (a.Lk + 512 / D - 1) / (512 / D);   // of 512 / D rows
 #define HIER_SEQ(G, LOOP) \
   hipLaunchKernelGGL((seq_kernel<D, NQ, G, LOOP, ONCE>), grid, block, 0, st, a, (uint32_t)nqg, (uint32_t)units)
@@ -541,14 +543,15 @@ extern "C" int hier_frame_attn(const HierFrameAttnArgs* args, void* stream) {
   HIER_REQUIRE(a.H <= 65535, HIER_EUNSUPPORTED, "at most 65535 heads");
   const int64_t q_tiles = ((int64_t)a.Lq + 127) / 128;
   const int64_t wgs = (int64_t)a.B * a.H * (use_seq(a) ? query_groups(a) : q_tiles);
-  HIER_REQUIRE(wgs <= hier::kMaxLaunchItems, HIER_EUNSUPPORTED, "too many queries");
+  const hier::Grid gr = hier::launch_grid(hier::xcd_grid(wgs), 256);
+  HIER_REQUIRE(wgs <= hier::kMaxLaunchItems && gr.x != 0, HIER_EUNSUPPORTED, "too many queries");
   const hipStream_t st = (hipStream_t)stream;
   if (use_seq(a)) {
     if (a.D == 128) launch_seq_d<128>(a, st);
     else launch_seq_d<64>(a, st);
     return hier::check_launch("seq_kernel");
   }
-  const dim3 grid((unsigned)hier::xcd_grid(wgs));
+  const dim3 grid(gr.x, gr.y);
   if (a.D == 128)
     hipLaunchKernelGGL(tile_kernel<128>, grid, dim3(256), 0, st, a, (int)q_tiles, (int)wgs);
   else

@@ -39,4 +39,19 @@ HIER_HD inline constexpr int xcd_logical(int bid, int grid) {
   return (bid % kXcds) * (grid / kXcds) + bid / kXcds;
 }
 
+// Grid of `blocks` workgroups of `threads`: a launch takes fewer than 2^32
+// threads along x, so more workgroups go over rows of a multiple of kXcds (bid =
+// y * x_size + x, handed out in that order).  Workgroups past `blocks` (up to
+// kXcds per row) return.  blocks <= 2^31; x = 0 if the grid would not fit an int.
+struct Grid {
+  uint32_t x, y;
+};
+HIER_HD inline constexpr Grid launch_grid(int64_t blocks, int threads) {
+  const int64_t row = ((1ll << 32) - 1) / threads / kXcds * kXcds;
+  if (blocks <= row) return {(uint32_t)blocks, 1u};
+  const int64_t y = (blocks + row - 1) / row;
+  const int64_t x = xcd_grid((blocks + y - 1) / y);
+  return x * y > 2147483647ll ? Grid{0u, 1u} : Grid{(uint32_t)x, (uint32_t)y};
+}
+
 }  // namespace hier

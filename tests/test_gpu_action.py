@@ -171,6 +171,24 @@ def test_frame_attention_weights_are_fp32(D, Lq):
     assert (err <= 2.0 ** -9 * ref.abs() + 2.0 ** -23).all(), float(err.max())
 
 
+@pytest.mark.parametrize("B,H,Lq", [(2_850_000, 24, 1), (16_800_000, 1, 17)])
+def test_frame_attention_many_sequences(B, H, Lq):
+    """More sequences and heads than a grid holds along x (2^26 waves; 2^24
+    matrix-tile workgroups): every one is computed.  Inputs are one sequence's,
+    expanded; one key, so the output is its V row."""
+    need_gpu()
+    say("frame attention many sequences", B, H, Lq)
+    D = 64
+    g = torch.Generator().manual_seed(H)
+    q, k, v = (torch.randn(1, L, H, D, generator=g).to("cuda", torch.bfloat16).expand(B, L, H, D)
+               for L in (Lq, 1, 1))
+    got = frame_attention(q, k, v, torch.zeros(Lq), torch.zeros(1), 1, -1)
+    torch.cuda.synchronize()
+    step = 9973
+    for part in (got[::step], got[-2:], got[B // 2:B // 2 + 2]):
+        assert torch.equal(part, v[:1].expand_as(part))
+
+
 class _Attn(nn.Module):
     """The attributes the reference's cached action attention reads."""
 

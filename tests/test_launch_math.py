@@ -6,7 +6,8 @@ workgroup id to logical item.  This test compiles that header with g++ and
 checks, for many item counts, that the grid is a multiple of the 8 XCDs and
 covers every item, that the map is a bijection on [0, grid), that every item
 below the count is run by exactly one workgroup (the others exit at the
-``logical >= total`` guard), and that consecutive logical items of one XCD's
+``logical >= total`` guard), that a grid of more threads than a launch takes
+along x goes over rows, and that consecutive logical items of one XCD's
 share are consecutive workgroups of that XCD (bid = 8 j + x).
 """
 
@@ -51,6 +52,20 @@ int main() {
   if (hier::xcd_grid(0) != 0 || hier::xcd_grid(-5) != 0) { printf("FAIL empty\n"); return 1; }
   // the largest accepted launch still has a grid that fits an int
   if (hier::xcd_grid(hier::kMaxLaunchItems) > 2147483647ll) { printf("FAIL max\n"); return 1; }
+  // a row stays below 2^32 threads and the rows hold every workgroup
+  for (int threads : {64, 256, 1024})
+    for (int64_t n : {(int64_t)1, (int64_t)7, (int64_t)1000003, (int64_t)16777208, (int64_t)16777215,
+                      (int64_t)16777216, (int64_t)16777217, (int64_t)67108864, (int64_t)100000007,
+                      (int64_t)2147470000}) {
+      const hier::Grid g = hier::launch_grid(n, threads);
+      if (g.x == 0 || (int64_t)g.x * threads > 4294967295ll || g.y > 65535 ||
+          (int64_t)g.x * g.y < n || (int64_t)g.x * g.y > 2147483647ll ||
+          (int64_t)g.x * g.y >= n + (int64_t)hier::kXcds * g.y + g.y || (g.y > 1 && g.x % hier::kXcds)) {
+        printf("FAIL rows n=%lld threads=%d x=%u y=%u\n", (long long)n, threads, g.x, g.y); return 1;
+      }
+      if (n % hier::kXcds == 0 && (int64_t)g.x * g.y % hier::kXcds) { printf("FAIL xcd rows\n"); return 1; }
+    }
+  if (hier::launch_grid(1ll << 31, 256).x != 0) { printf("FAIL int\n"); return 1; }
   printf("OK\n");
   return 0;
 }
@@ -75,3 +90,5 @@ def test_kernels_use_the_shared_launch_math():
         assert "hier_launch.h" in text, name
         assert "bid & 7" not in text and "+ 7) / 8 * 8" not in text, name
         assert "xcd_logical(blockIdx.x, gridDim.x)" in text, name
+    text = (CSRC / "hier_frame_attn.hip").read_text()
+    assert text.count("launch_grid(") == 2 and "xcd_logical((int)(blockIdx.y" in text
