@@ -226,8 +226,14 @@ def check(rc: int, what: str) -> None:
 
 
 def stream_of(device) -> int:
-    """The handle of PyTorch's current stream on ``device`` (asked per call;
-    without the stream object that ``torch.cuda.current_stream`` makes, 6 us)."""
+    """The handle of PyTorch's current stream on ``device``, a GPU (a launch
+    handed host pointers would fault it): the number that
+    ``torch.cuda.current_stream(device).cuda_stream`` gives, without the
+    stream object."""
+    if type(device) is not torch.device:
+        device = torch.device("cuda", device) if isinstance(device, int) else torch.device(device)
+    if device.type != "cuda":
+        raise ValueError(f"expected a GPU, got device {device}")
     index = device.index
     return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if index is None else index)
 

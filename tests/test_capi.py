@@ -8,6 +8,7 @@ import subprocess
 from pathlib import Path
 
 import pytest
+import torch
 
 from multics_amd import _capi
 
@@ -27,6 +28,7 @@ STRUCTS = {
     "HierSteReduceArgs": _capi.HierSteReduceArgs,
     "HierMembershipArgs": _capi.HierMembershipArgs,
     "HierPrologueBwdArgs": _capi.HierPrologueBwdArgs,
+    "HierPrologueGradArgs": _capi.HierPrologueGradArgs,
     "HierMergeArgs": _capi.HierMergeArgs,
     "HierTrimArgs": _capi.HierTrimArgs,
 }
@@ -124,3 +126,32 @@ def test_forward_rejects_views_past_the_24_bit_row_limit_without_a_gpu():
     assert b"2^24" in lib.hier_last_error()
     a.kv_rows = 1 << 24
     assert lib.hier_attn_fwd(C.byref(a), None) == _capi.HIER_OK
+
+
+@pytest.mark.parametrize("device", ["cpu", torch.device("cpu"), torch.device("meta")])
+def test_a_stream_is_a_gpu_stream(device):
+    with pytest.raises(ValueError, match="expected a GPU"):
+        _capi.stream_of(device)
+
+
+def test_host_tensors_reach_no_launch(monkeypatch):
+    """Entry points that look at no tensor's device themselves refuse host
+    tensors before they launch (a kernel would read host pointers)."""
+    from multics_amd import kernels
+    from multics_amd.paged_cache import HierPagedKVCache
+    monkeypatch.setattr(_capi, "call", lambda *a: pytest.fail("launched on host tensors"))
+    c = HierPagedKVCache(num_players=2, num_groups=1, num_patches=4, num_local_hub_tokens=1,
+                         num_global_hub_tokens=1, num_heads=1, head_dim=64, local_attn_size=1,
+                         num_frame_per_block=1, device="cpu")
+    kv = torch.zeros(2 * 4 + 2, 1, 64, dtype=torch.bfloat16)
+    with pytest.raises(ValueError, match="expected a GPU"):
+        c.append(kv, kv, 0, 1, [[True]])
+    x, w = torch.zeros(3, 512, dtype=torch.bfloat16), torch.ones(512, dtype=torch.bfloat16)
+    cs = torch.ones(3, 32)
+    with pytest.raises(ValueError, match="expected a GPU"):
+        kernels.qkv_prologue(x, x, None, norm_q_w=w, norm_k_w=w, rope_cos=cs, rope_sin=cs,
+                             num_heads=8, eps=1e-6)
+    q = x.requires_grad_()
+    with pytest.raises(ValueError, match="expected a GPU"):
+        kernels.qk_prologue_train(q, q, norm_q_w=w, norm_k_w=w, rope_cos=cs, rope_sin=cs,
+                                  num_heads=8, eps=1e-6)
