@@ -1680,15 +1680,21 @@ def cached_tiles(*, device, P, N, L, KL, KG, n_frames, n_block, local_attn, fram
            bool(direct_player), no_local, _freeze(membership), _freeze(global_only))
     hit = _lru_get(_META_CACHE, key)
     if hit is None:
-        topo = cached_topology(
-            P=P, N=N, L=L, KL=KL, KG=KG, n_frames=n_frames, n_block=n_block, local_attn=local_attn,
-            agent_frame_lists=[fr] * P, local_frame_lists=[] if no_local else [fr] * N,
-            global_frame_list=fr if KG > 0 else (), local_active_frames=local_active_frames,
-            labels=labels, q_active=q_active, direct_player=direct_player, membership=membership,
-            global_only=global_only, hier_no_local_hub=no_local, tile_bases=tile_bases)
-        hit = build(topo, device).tiles
+        hit = _paged_tiles(device=device, P=P, N=N, L=L, KL=KL, KG=KG, n_frames=n_frames,
+                           n_block=n_block, local_attn=local_attn, fr=fr, tile_bases=tile_bases,
+                           local_active_frames=local_active_frames, labels=labels,
+                           q_active=q_active, direct_player=direct_player, membership=membership,
+                           global_only=global_only, no_local=no_local)
         _lru_put(_META_CACHE, key, hit, "WAN_HIER_SEGMENTED_META_CACHE_SIZE", "64")
     return hit
+
+
+def _paged_tiles(*, device, P, N, KG, fr, no_local, **topology) -> TileList:
+    topo = cached_topology(P=P, N=N, KG=KG, agent_frame_lists=[fr] * P,
+                           local_frame_lists=[] if no_local else [fr] * N,
+                           global_frame_list=fr if KG > 0 else (), hier_no_local_hub=no_local,
+                           **topology)
+    return build(topo, device).tiles
 
 
 def cached_window_tiles(cache, end_frame: int, *, device, n_frames, n_block, local_attn, labels,
@@ -1697,8 +1703,9 @@ def cached_window_tiles(cache, end_frame: int, *, device, n_frames, n_block, loc
     """``cached_tiles`` over the window that a ``HierPagedKVCache`` holds for a
     block ending at ``end_frame``.  The list is kept under what the window is
     made of -- the cache's shape, its ring and its local-hub flags -- beside the
-    block's topology (host arrays), in the same LRU, so the later passes over a
-    block neither gather its pages nor hash them."""
+    block's topology (host arrays), in the same LRU (there only, an entry per
+    window), so the later passes over a block neither gather its pages nor hash
+    them."""
     raw = lambda x: None if x is None else (np.shape(x), np.asarray(x).tobytes())
     key = ("window", str(device), cache.P, cache.N, cache.L, cache.KL, cache.KG, cache.R,
            cache.no_local, int(end_frame), cache.slot_frame.tobytes(),
@@ -1708,12 +1715,12 @@ def cached_window_tiles(cache, end_frame: int, *, device, n_frames, n_block, loc
     if hit is None:
         frames, bases, lact = cache.window(end_frame)
         listed = lambda x: None if x is None else np.asarray(x).tolist()
-        hit = cached_tiles(
+        hit = _paged_tiles(
             device=device, P=cache.P, N=cache.N, L=cache.L, KL=cache.KL, KG=cache.KG,
-            n_frames=n_frames, n_block=n_block, local_attn=local_attn, frames=frames,
+            n_frames=n_frames, n_block=n_block, local_attn=local_attn, fr=tuple(frames),
             tile_bases=bases, local_active_frames=lact, labels=listed(labels),
             q_active=listed(q_active), direct_player=direct_player, membership=membership,
-            global_only=global_only, hier_no_local_hub=hier_no_local_hub)
+            global_only=global_only, no_local=bool(hier_no_local_hub))
         _lru_put(_META_CACHE, key, hit, "WAN_HIER_SEGMENTED_META_CACHE_SIZE", "64")
     return hit
 

@@ -91,3 +91,33 @@ def test_cached_paths_refuse_autograd():
     q = torch.zeros(1, 3, 1, 64, requires_grad=True)
     with pytest.raises(RuntimeError, match="inference-only"):
         frame_attention(q, q, q, torch.arange(3), torch.arange(3), 3, -1)
+
+
+def test_a_window_list_takes_one_entry(monkeypatch):
+    """The LRU of window lists holds as many windows as its size says: as
+    many rollouts taking turns build each list once, one more than that
+    evicts the oldest."""
+    from types import SimpleNamespace
+
+    from multics_amd import metadata as M
+    built = []
+    monkeypatch.setattr(M, "build", lambda topo, device: SimpleNamespace(
+        tiles=built.append(topo) or SimpleNamespace()))
+    monkeypatch.setattr(M, "_META_CACHE", type(M._META_CACHE)())
+    monkeypatch.setenv("WAN_HIER_SEGMENTED_META_CACHE_SIZE", "4")
+    c = _cache()
+    act = np.ones((2, 2), bool)
+
+    def tiles(f0):
+        c.reset()
+        for f in range(max(0, f0 + 2 - c.R), f0 + 2):
+            c.slot_frame[f % c.R] = f
+            c.local_active[:, f % c.R] = True
+        return M.cached_window_tiles(c, f0 + 1, device="cpu", n_frames=2, n_block=2, local_attn=4,
+                                     labels=np.zeros((2, 3), np.int64), q_active=act,
+                                     direct_player=True)
+
+    first = [tiles(f) for f in (0, 2, 4, 6)]
+    assert [tiles(f) for f in (0, 2, 4, 6)] == first and len(built) == 4
+    tiles(8)
+    assert len(built) == 5 and tiles(2) is first[1] and tiles(0) is not first[0]
