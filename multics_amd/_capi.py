@@ -225,13 +225,11 @@ def check(rc: int, what: str) -> None:
     raise RuntimeError(msg)
 
 
-def stream_of(device) -> int:
-    """The handle of PyTorch's current stream on ``device``, a GPU (a launch
+def stream_of(device: torch.device) -> int:
+    """The handle of PyTorch's current stream on ``device``, a GPU's (a launch
     handed host pointers would fault it): the number that
     ``torch.cuda.current_stream(device).cuda_stream`` gives, without the
     stream object."""
-    if type(device) is not torch.device:
-        device = torch.device("cuda", device) if isinstance(device, int) else torch.device(device)
     if device.type != "cuda":
         raise ValueError(f"expected a GPU, got device {device}")
     index = device.index

@@ -22,8 +22,7 @@ from .module import rope_apply
 from .rolling import rolling_cache_append  # noqa: F401  (re-exported)
 
 
-def _stream(dev) -> C.c_void_p:
-    return C.c_void_p(_capi.stream_of(dev))
+_stream = _capi.stream_of
 
 
 def ensure_action_cache(parent: dict, name: str, batch: int, n_heads: int, head_dim: int,

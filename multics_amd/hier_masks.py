@@ -29,6 +29,7 @@ from typing import Optional
 import numpy as np
 import torch
 
+from . import _ready
 from . import metadata as M
 from .metadata import TileList, _freeze
 from .topology import (_prepare_hier_group_tensors, _prepare_hier_membership_tensors,
@@ -63,15 +64,14 @@ _MASK_CACHE: "OrderedDict[tuple, tuple]" = OrderedDict()
 
 def _cache_put(key, value):
     n = int(os.environ.get("WAN_HIER_BLOCKMASK_CACHE_SIZE", "2"))
-    if n < 0:
-        _MASK_CACHE[key] = value
+    if n == 0 or _ready.being_captured(value):
         return value
-    if n == 0:
-        return value
-    _MASK_CACHE[key] = value
-    _MASK_CACHE.move_to_end(key)
-    while len(_MASK_CACHE) > n:
-        _MASK_CACHE.popitem(last=False)
+    ready = _ready.made(value)
+    with _ready.LOCK:
+        _MASK_CACHE[key] = (value, ready)
+        _MASK_CACHE.move_to_end(key)
+        while 0 < n < len(_MASK_CACHE):
+            _MASK_CACHE.popitem(last=False)
     return value
 
 
@@ -114,9 +114,8 @@ def build_stage2_hier_flex_block_mask(num_players: int, num_frames: int, num_pat
     key = ("hier", P, T, L, N, KL, KG, int(num_frame_per_block), int(local_attn_size),
            bool(direct_player), bool(hier_no_local_hub), _freeze(labels_np), _freeze(mem_np),
            _freeze(go_np), _freeze(act_np), S_pad, str(torch.device(device)))
-    hit = _MASK_CACHE.get(key)
+    hit = M._lru_get(_MASK_CACHE, key)
     if hit is not None:
-        _MASK_CACHE.move_to_end(key)
         return hit
     tiles = M.full_sequence_tiles(
         device=device, P=P, T=T, L=L, N=N, KL=KL, KG=KG, n=int(num_frame_per_block),

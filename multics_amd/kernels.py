@@ -20,8 +20,7 @@ from . import metadata as M
 from .metadata import HierTiledBlockLayout, TileList, backward_lists, folded_key_list
 
 
-def _stream(dev) -> C.c_void_p:
-    return C.c_void_p(_capi.stream_of(dev))
+_stream = _capi.stream_of
 
 
 def _rows_view(t: torch.Tensor):

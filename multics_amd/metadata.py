@@ -25,6 +25,7 @@ from __future__ import annotations
 import ctypes as C
 import dataclasses
 import os
+import threading
 import weakref
 from collections import OrderedDict
 from dataclasses import dataclass, field
@@ -33,7 +34,7 @@ from typing import Optional
 import numpy as np
 import torch
 
-from . import _capi
+from . import _capi, _ready
 
 TILE_KEYS = 64          # attention kernel key tile
 ROWS_PER_ITEM = 128     # attention kernel query rows per work item (4 waves x 32)
@@ -88,6 +89,39 @@ class TileList:
     fwd_items: Optional[torch.Tensor] = None
     fwd_n_items: int = 0
     row_table: Optional[torch.Tensor] = None
+
+    def kept_tensors(self):
+        """The list's tensors and those of its launch list."""
+        run = self.__dict__.get("_launch")
+        return [self.items, self.kv_idx, self.kv_mask, self.blk_and, self.fwd_items,
+                self.row_table] + ([] if run is None else [run.items, run.fwd_items])
+
+
+# Lists derived from a list are kept on it, made on the stream that first asks
+# for them.  ``_ready`` of a built list is the event behind its build, of a
+# derived one the event behind its derivation; a derived list without one of its own
+# shares its source's (made in the same call, as those of a training step's
+# list are, which nobody keeps).
+
+def _derived_on(source: TileList, piece: TileList) -> TileList:
+    """``piece``, just derived from ``source`` by launches on the current stream."""
+    if source.__dict__.get("_ready") is not None and _keeps(source):
+        piece.__dict__["_ready"] = _ready.made(piece)
+    return piece
+
+
+def _use_derived(source: TileList, piece: TileList, value=None) -> None:
+    """The current stream may use ``piece`` (``value``: with what came with
+    it), found on ``source``."""
+    ready = piece.__dict__.get("_ready")
+    if ready is not None and ready is not source.__dict__.get("_ready"):
+        ready.join(piece if value is None else value)
+
+
+def _keeps(source: TileList) -> bool:
+    """Whether a piece derived now may stay on ``source``: not under graph
+    capture, unless the capture makes ``source`` too."""
+    return source.__dict__.get("_ready") is None or not _ready.capturing(source.items.device)
 
 
 @dataclass(frozen=True)
@@ -648,9 +682,10 @@ class _HubMerge:
             self.fwd_n_items = len(idx)
             self.row_table = torch.tensor(rows_tab, dtype=torch.int32, device=dev).reshape(-1, 2)
 
-    def run(self, items, kv_idx, kv_mask, blk_and, n_items: int, stream):
+    def run(self, items, kv_idx, kv_mask, blk_and, n_items: int, stream, acc=None):
         """Merged lists into their slots; the shared list's items and the
-        forward list's items (None without folded rows)."""
+        forward list's items (None without folded rows).  ``acc``: the
+        workspace (default: the object's own)."""
         # with merged hub items only (none folded), they take the place of the
         # hub items they replace, in front of the players' (the scatter, which
         # reads those, has run by then): the shared list is a slice
@@ -662,7 +697,7 @@ class _HubMerge:
         a = _capi.HierMergeArgs(
             n_groups=self.n_all_groups, n_src=self.n_src, rows=self.rows, rows_per_item=self.rpi,
             items=items.data_ptr(), kv_idx=kv_idx.data_ptr(), kv_mask=kv_mask.data_ptr(),
-            blk_and=blk_and.data_ptr(), acc=self.acc.data_ptr(),
+            blk_and=blk_and.data_ptr(), acc=(self.acc if acc is None else acc).data_ptr(),
             **{k: v.data_ptr() for k, v in d.items()}, out_items=out.data_ptr())
         _capi.call("hier_merge_hub_lists", C.byref(a), stream)
         if in_place:
@@ -876,7 +911,8 @@ def build(topo: BlockTopology, device, *, segmented_block_m: Optional[int] = Non
     # the fold plan, which the key-major list can take too (folded_key_list)
     tiles._fold = merge if merge is not None and merge.key_fold else None
     tiles._layout = (tile_off[:-1].copy(), item_start.reshape(-1).copy())   # per (block, stream)
-    launch_list(tiles)
+    run = launch_list(tiles)
+    tiles.__dict__["_ready"] = run.__dict__["_ready"] = _ready.made(tiles)
     layouts = None
     if tiled_res is not None:
         layouts = [HierTiledBlockLayout(tiles=tiles, block=b, **d) for b, d in enumerate(tiled_res)]
@@ -1114,7 +1150,10 @@ def ste_classes(tiles: TileList, ste_geometry):
     cache = tiles.__dict__.setdefault("_ste_classes", {})
     hit = cache.get(key)
     if hit is not None:
-        return hit
+        res, ready = hit
+        if ready is not None:
+            ready.join(res)
+        return res
     if not tiles.items.is_cuda:
         raise NotImplementedError("ste_classes builds on the GPU; use ste_classes_host")
     P, T, L, N, KL = key
@@ -1126,8 +1165,10 @@ def ste_classes(tiles: TileList, ste_geometry):
     first = torch.empty(max(tiles.n_items, 1), dtype=torch.int32, device=tiles.items.device)
     _capi.call("hier_derive_ste_classes", C.byref(a), cls.data_ptr(), first.data_ptr(),
                _capi.stream_of(tiles.items.device))
-    cache[key] = (cls, first)
-    return cache[key]
+    if _keeps(tiles):
+        kept = tiles.__dict__.get("_ready") is not None
+        cache[key] = ((cls, first), _ready.made(cls) if kept else None)
+    return cls, first
 
 
 _DERIVE_ERRORS = ((1, "a token is a query row of two groups"),
@@ -1215,6 +1256,7 @@ def folded_key_list(tiles: TileList, kt: TileList) -> TileList:
         return kt
     hit = kt.__dict__.get("_folded")
     if hit is not None:
+        _use_derived(kt, hit)
         return hit
     dev = kt.items.device
     sizes = kt.items[:kt.n_items, 6].cpu().numpy().astype(np.int64)
@@ -1263,8 +1305,9 @@ def folded_key_list(tiles: TileList, kt: TileList) -> TileList:
     folded = dataclasses.replace(kt, items=items, n_items=int(items.shape[0]), kv_idx=kv_idx,
                                  kv_mask=kv_mask, blk_and=blk, row_table=tiles.row_table)
     folded._keepalive = (acc, d)
+    run = launch_list(folded)
+    run.__dict__["_ready"] = _derived_on(kt, folded).__dict__.get("_ready")
     kt.__dict__["_folded"] = folded
-    launch_list(folded)
     return folded
 
 
@@ -1279,9 +1322,11 @@ def backward_lists(tiles: TileList, ste_geometry=None):
     cache = tiles.__dict__.setdefault("_derived", {})
     hit = cache.get(key)
     if hit is not None:
+        _use_derived(tiles, hit[0], hit)
         return hit
     if tiles.items.is_cuda:
         res = _derive_device(tiles, key)
+        launch_list(res[0]).__dict__["_ready"] = _derived_on(tiles, res[0]).__dict__.get("_ready")
     else:
         kt = next(iter(cache.values()))[0] if cache else transpose_tiles_host(tiles)
         ste = None if key is None else ste_tiles_host(tiles, P=key[0], T=key[1], L=key[2],
@@ -1319,6 +1364,7 @@ def launch_list(tiles: TileList) -> TileList:
         return tiles
     hit = tiles.__dict__.get("_launch")
     if hit is not None:
+        _use_derived(tiles, hit)
         return hit
     if not tiles.items.is_cuda:
         return tiles
@@ -1349,7 +1395,9 @@ def _set_launch(tiles: TileList, items: torch.Tensor, fwd: Optional[torch.Tensor
     # is freed when its last user drops it, without the cycle collector
     run.__dict__["_is_launch"] = True
     run.__dict__["_source"] = weakref.ref(tiles)
-    tiles.__dict__["_launch"] = run
+    _derived_on(tiles, run)
+    if _keeps(tiles):
+        tiles.__dict__["_launch"] = run
     return run
 
 
@@ -1369,8 +1417,9 @@ def launch_ste_first(tiles: TileList, ste_geometry) -> tuple:
 
 def transpose_tiles(tiles: TileList) -> TileList:
     """Key-major list of ``tiles`` (see ``backward_lists``), cached on it."""
-    for (kt, _) in getattr(tiles, "_derived", {}).values():
-        return kt
+    for hit in getattr(tiles, "_derived", {}).values():
+        _use_derived(tiles, hit[0], hit)
+        return hit[0]
     return backward_lists(tiles)[0]
 
 
@@ -1388,20 +1437,29 @@ _LAYOUT_CACHE: "OrderedDict[tuple, object]" = OrderedDict()
 
 
 def _lru_get(cache, key):
-    v = cache.get(key)
-    if v is not None:
+    """The kept value, for use on the current stream."""
+    with _ready.LOCK:
+        hit = cache.get(key)
+        if hit is None:
+            return None
         cache.move_to_end(key)
-    return v
+    value, ready = hit
+    if ready is not None:
+        ready.join(value)
+    return value
 
 
 def _lru_put(cache, key, value, env, default):
+    """Keeps a value that launches on the current stream have just made."""
     n = max(int(os.environ.get(env, default)), 0)
-    if n == 0:
+    if n == 0 or _ready.being_captured(value):
         return
-    cache[key] = value
-    cache.move_to_end(key)
-    while len(cache) > n:
-        cache.popitem(last=False)
+    ready = _ready.made(value)
+    with _ready.LOCK:
+        cache[key] = (value, ready)
+        cache.move_to_end(key)
+        while len(cache) > n:
+            cache.popitem(last=False)
 
 
 def _freeze(x):
@@ -1514,6 +1572,34 @@ def full_sequence_tiles(*, device, P, T, L, N, KL, KG, n, window, direct, labels
     return hit
 
 
+_PLAN_STREAMS = 8       # streams whose step buffers a plan keeps
+
+
+class _StepBuffers:
+    """What a step writes before its lists: the topology arrays of the
+    logits and the workspaces of the list passes, for one stream."""
+
+    def __init__(self, plan):
+        P, T, N, n, dev = plan.P, plan.T, plan.N, plan.n, plan.device
+        B = T // n
+        u8 = dict(dtype=torch.uint8, device=dev)
+        self.mem = torch.zeros((T, N, P), **u8)
+        self.go = torch.zeros((T, P), **u8)
+        self.la = torch.zeros((B, max(N, 1), max(plan.fl_max, 1)), **u8)
+        self.qa = torch.zeros((B, n, max(N, 1)), **u8)
+        self.ws = torch.empty(plan.ws_bytes, **u8)
+        self.totals = torch.zeros(8, dtype=torch.int64, device=dev)
+        merge = getattr(plan.sup, "_merge", None)
+        self.acc = None if merge is None else torch.empty_like(merge.acc)
+        self.margs = _capi.HierMembershipArgs(
+            T=T, N=N, P=P, B=B, n=n, fl_max=plan.fl_max, la_frame=plan.la_frame.data_ptr(),
+            membership=self.mem.data_ptr(), global_only=self.go.data_ptr(),
+            q_active=self.qa.data_ptr(), local_active=self.la.data_ptr())
+        self.t = type(plan.t).from_buffer_copy(plan.t)
+        self.t.membership, self.t.global_only = self.mem.data_ptr(), self.go.data_ptr()
+        self.t.local_active, self.t.q_active = self.la.data_ptr(), self.qa.data_ptr()
+
+
 class MembershipLogitsPlan:
     """Per-step lists of a full-sequence membership topology whose membership
     is ``logits > 0`` of soft logits on the device -- the training case, where
@@ -1536,7 +1622,11 @@ class MembershipLogitsPlan:
       * runs ``hier_derive_count`` / ``hier_derive_build`` into the bounded
         key-major arrays (offsets scanned on the device),
     all asynchronous on the current stream.  ``logical_pairs`` of a step's
-    list is -1 (not counted: that would need a read-back)."""
+    list is -1 (not counted: that would need a read-back).
+
+    Every stream that steps has buffers of its own (``_StepBuffers``), so
+    steps of one geometry on several streams do not write over each other;
+    threads take turns to issue a step."""
 
     def __init__(self, *, device, P, T, L, N, KL, KG, n, window, direct, no_local=False):
         dev = torch.device(device)
@@ -1548,26 +1638,16 @@ class MembershipLogitsPlan:
         # no folded rows: which players' rows join which hub changes with the logits
         sup = build(sup_topo, dev, fold_tails=False).tiles
         self.t, self._static = _topo_struct(sup_topo, dev)
-        B = T // n
-        fl_max = int(self.t.fl_max)
-        u8 = dict(dtype=torch.uint8, device=dev)
-        self.mem = torch.zeros((T, N, P), **u8)
-        self.go = torch.zeros((T, P), **u8)
-        self.la = torch.zeros((B, max(N, 1), max(fl_max, 1)), **u8)
-        self.qa = torch.zeros((B, n, max(N, 1)), **u8)
+        self.fl_max = int(self.t.fl_max)
         # frame of local-slot column fi of block b (padding: valid = 0)
-        kf = np.full((B, max(fl_max, 1)), -1, np.int32)
+        B = T // n
+        kf = np.full((B, max(self.fl_max, 1)), -1, np.int32)
         if not no_local:
             for b in range(B):
                 fr = sup_topo.local_frames[b][0]
                 kf[b, :len(fr)] = fr
         self.la_frame = torch.from_numpy(kf).to(dev)
-        self._margs = _capi.HierMembershipArgs(
-            T=T, N=N, P=P, B=B, n=n, fl_max=fl_max, la_frame=self.la_frame.data_ptr(),
-            membership=self.mem.data_ptr(), global_only=self.go.data_ptr(),
-            q_active=self.qa.data_ptr(), local_active=self.la.data_ptr())
-        self.t.membership, self.t.global_only = self.mem.data_ptr(), self.go.data_ptr()
-        self.t.local_active, self.t.q_active = self.la.data_ptr(), self.qa.data_ptr()
+        self.device = self.la_frame.device
         tile_off, item_start = sup._layout          # the builder reads int64 / int32
         self._kv_off = torch.from_numpy(tile_off.astype(np.int64)).to(dev)
         self._item_off = torch.from_numpy(item_start.astype(np.int32)).to(dev)
@@ -1577,10 +1657,30 @@ class MembershipLogitsPlan:
         kt_sup, _ = backward_lists(sup, None)
         self.key_cap = int(kt_sup.kv_idx.numel())
         self.n_groups, self.nq = _groups_and_frames(sup)
-        a = self._derive_args(sup)
-        self.ws = torch.empty(max(int(_capi.lib().hier_derive_workspace(C.byref(a))), 1),
-                              dtype=torch.uint8, device=dev)
-        self.totals = torch.zeros(8, dtype=torch.int64, device=dev)
+        self.ws_bytes = max(int(_capi.lib().hier_derive_workspace(C.byref(self._derive_args(sup)))), 1)
+        self._steps: "OrderedDict[int, _StepBuffers]" = OrderedDict()   # by stream
+        self._lock = threading.Lock()
+        self._ready = _ready.made(self)
+
+    def kept_tensors(self):
+        """What the steps of every stream read."""
+        merge = getattr(self.sup, "_merge", None)
+        return [self.la_frame, self._kv_off, self._item_off, self._static, self.sup] + \
+            ([] if merge is None else [merge._dev])
+
+    def _buffers(self, stream: int) -> "_StepBuffers":
+        """The buffers of a step on the current stream: the stream's own,
+        kept for its next step.  A graph under capture gets buffers of its
+        own, which live as long as the lists it makes."""
+        if _ready.capturing(self.device):
+            return _StepBuffers(self)
+        buf = self._steps.get(stream)
+        if buf is None:
+            buf = self._steps[stream] = _StepBuffers(self)
+        self._steps.move_to_end(stream)
+        while len(self._steps) > _PLAN_STREAMS:
+            self._steps.popitem(last=False)
+        return buf
 
     def _derive_args(self, tiles: TileList):
         # no STE geometry: the key-major list only (the dQ pass takes the
@@ -1594,14 +1694,21 @@ class MembershipLogitsPlan:
     def build(self, logits: torch.Tensor) -> TileList:
         """The forward tile list of ``logits > 0`` ([T, N, P]) with its
         key-major list cached on it (``backward_lists``)."""
-        P, T, N, n = self.P, self.T, self.N, self.n
-        dev = self.mem.device
+        P, T, N = self.P, self.T, self.N
+        dev = self.device
         if tuple(logits.shape) != (T, N, P):
             raise ValueError(f"membership logits must be [T,N,P] = {(T, N, P)}")
+        with self._lock:
+            return self._build(logits, dev)
+
+    def _build(self, logits: torch.Tensor, dev) -> TileList:
         lg = logits.detach().to(device=dev, dtype=torch.float32).contiguous()
         stream = _capi.stream_of(dev)
-        self._margs.logits = lg.data_ptr()
-        _capi.call("hier_membership_from_logits", C.byref(self._margs), stream)
+        if self._ready is not None:
+            self._ready.join(self)
+        buf = self._buffers(stream)
+        buf.margs.logits = lg.data_ptr()
+        _capi.call("hier_membership_from_logits", C.byref(buf.margs), stream)
         sup = self.sup
         i32 = dict(dtype=torch.int32, device=dev)
         merge = getattr(sup, "_merge", None)
@@ -1615,9 +1722,9 @@ class MembershipLogitsPlan:
         out.tile_item_off = self._item_off.data_ptr()
         out.tile_kv_idx, out.tile_kv_mask = kv_idx.data_ptr(), kv_mask.data_ptr()
         out.tile_blk_and, out.tile_items = blk.data_ptr(), items.data_ptr()
-        _capi.call("hier_meta_build", C.byref(self.t), C.byref(out), stream)
+        _capi.call("hier_meta_build", C.byref(buf.t), C.byref(out), stream)
         if merge is not None:
-            items, _ = merge.run(items, kv_idx, kv_mask, blk, n_pre, stream)
+            items, _ = merge.run(items, kv_idx, kv_mask, blk, n_pre, stream, buf.acc)
         tiles = TileList(items=items, kv_idx=kv_idx, kv_mask=kv_mask, blk_and=blk,
                          n_items=sup.n_items, item_ranges=sup.item_ranges, logical_pairs=-1,
                          key_extent=sup.key_extent, row_extent=sup.row_extent,
@@ -1626,7 +1733,7 @@ class MembershipLogitsPlan:
                          merged_blocks=sup.merged_blocks)
         # key-major list, sized by the superset's
         a = self._derive_args(tiles)
-        a.ws, a.ws_bytes, a.totals = self.ws.data_ptr(), int(self.ws.numel()), self.totals.data_ptr()
+        a.ws, a.ws_bytes, a.totals = buf.ws.data_ptr(), self.ws_bytes, buf.totals.data_ptr()
         k_items = torch.empty((sup.n_items, 8), **i32)
         k_idx = torch.empty(max(self.key_cap, 1), **i32)
         k_mask = torch.empty(max(self.key_cap, 1), **i32)
@@ -1643,7 +1750,7 @@ class MembershipLogitsPlan:
                       n_groups=sup.n_groups, frames_per_group=sup.frames_per_group,
                       merged_blocks=sup.merged_blocks)
         tiles.__dict__["_derived"] = {None: (kt, None)}
-        tiles._keepalive = (self, a, lg)
+        tiles._keepalive = (self, buf, a, lg)
         _launch_pair(tiles, kt)
         return tiles
 

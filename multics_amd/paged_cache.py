@@ -32,8 +32,7 @@ import torch
 from . import _capi
 
 
-def _stream(dev) -> C.c_void_p:
-    return C.c_void_p(_capi.stream_of(dev))
+_stream = _capi.stream_of
 
 
 class HierPagedKVCache:

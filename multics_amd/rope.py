@@ -19,6 +19,8 @@ from typing import Tuple
 
 import torch
 
+from . import _capi, _ready
+
 WAN_REROPE_SPLITS = (12, 32, 42, 42)   # rope.py:5
 
 
@@ -120,7 +122,9 @@ def build_self_attn_freqs_with_hub(freqs_bands, simplex_vertices, f, h, w, devic
 # The last tables converted: every layer of a model step receives the same
 # complex table, so the conversion runs once per step, not once per layer.
 # An entry holds its table (its storage cannot be reused while the entry
-# lives) and the table's version counter (an in-place change is a miss).
+# lives) and the table's version counter (an in-place change is a miss), and is
+# for the stream that made it; one made under graph capture holds nothing until
+# the graph runs and is not kept.
 _COS_SIN_CACHE: "OrderedDict[tuple, tuple]" = OrderedDict()
 _COS_SIN_CACHE_SIZE = 2
 
@@ -128,19 +132,21 @@ _COS_SIN_CACHE_SIZE = 2
 def freqs_to_cos_sin(freqs: torch.Tensor, device=None):
     """``[S,1,D/2]`` (or ``[S,D/2]``) complex table -> fp32 (cos, sin) ``[S,D/2]`` on ``device``.
     The result of the last tables is cached (keyed by the table object, its
-    version counter and the device)."""
+    version counter, the device and the stream)."""
     dev = torch.device(device) if device is not None else freqs.device
-    key = (id(freqs), freqs._version, str(dev))
-    hit = _COS_SIN_CACHE.get(key)
-    if hit is not None and hit[0] is freqs:
-        _COS_SIN_CACHE.move_to_end(key)
-        return hit[1], hit[2]
+    key = (id(freqs), freqs._version, str(dev), _capi.stream_of(dev) if dev.type == "cuda" else 0)
+    with _ready.LOCK:
+        hit = _COS_SIN_CACHE.get(key)
+        if hit is not None and hit[0] is freqs:
+            _COS_SIN_CACHE.move_to_end(key)
+            return hit[1], hit[2]
     f = freqs.reshape(freqs.shape[0], -1)
     if device is not None:
         f = f.to(device)
     cs, sn = f.real.to(torch.float32).contiguous(), f.imag.to(torch.float32).contiguous()
-    if not freqs.requires_grad:
-        _COS_SIN_CACHE[key] = (freqs, cs, sn)
-        while len(_COS_SIN_CACHE) > _COS_SIN_CACHE_SIZE:
-            _COS_SIN_CACHE.popitem(last=False)
+    if not freqs.requires_grad and not _ready.capturing(dev):
+        with _ready.LOCK:
+            _COS_SIN_CACHE[key] = (freqs, cs, sn)
+            while len(_COS_SIN_CACHE) > _COS_SIN_CACHE_SIZE:
+                _COS_SIN_CACHE.popitem(last=False)
     return cs, sn

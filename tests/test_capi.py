@@ -128,7 +128,7 @@ def test_forward_rejects_views_past_the_24_bit_row_limit_without_a_gpu():
     assert lib.hier_attn_fwd(C.byref(a), None) == _capi.HIER_OK
 
 
-@pytest.mark.parametrize("device", ["cpu", torch.device("cpu"), torch.device("meta")])
+@pytest.mark.parametrize("device", [torch.device("cpu"), torch.device("cpu", 0), torch.device("meta")])
 def test_a_stream_is_a_gpu_stream(device):
     with pytest.raises(ValueError, match="expected a GPU"):
         _capi.stream_of(device)
