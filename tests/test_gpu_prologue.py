@@ -223,14 +223,19 @@ def test_prologue_backward_matches_fp32_autograd(camera, shape):
     (1100, 24, 128, 220),    # 9 tokens per workgroup: a ragged last trip in each
     (70, 28, 128, 5),        # 8 channels per thread, two tokens per trip, odd runs
     (70, 64, 64, 70),        # the largest model dim
+    (1536, 24, 128, 1),      # 12 tokens and camera rows per workgroup: its slots just hold them
+    (1664, 24, 128, 1),      # 13: the row past the slots is the last token's
+    (1700, 24, 128, 1),      # 14: one row more, and a last workgroup of 6
+    (3200, 24, 128, 1),      # 25: as many rows again after the slots are full
+    (3200, 24, 128, 2),      # 13 rows of two tokens, runs that cross workgroups
 ])
 def test_prologue_backward_sums(S, H, D, run):
     """The sums over tokens of the prologue backward (gain and camera-weight
     gradients) and the projections' gradients, where the token split, the
     trips and the camera runs (``run`` tokens of one row, every third run
     zeros) can go wrong, against float64 autograd.  Bounds: results are bf16
-    (2^-9 of the value) of fp32 sums of terms with the forward's bf16 rounding
-    of a (2^-9 of each term): 1 % of the largest entry."""
+    (2^-8 of the value) of fp32 sums of terms with the forward's bf16 rounding
+    of a (2^-8 of each term): 1 % of the largest entry."""
     need_gpu()
     from multics_amd.kernels import qk_prologue_train
     say("prologue backward sums", S, H, D, run)
@@ -269,3 +274,88 @@ def test_prologue_backward_sums(S, H, D, run):
         err = (a.double().cpu() - b).abs().max().item()
         say(f"  {name}: max-abs {err:.3e} of {b.abs().max().item():.3e}")
         assert err <= 1e-2 * b.abs().max().item(), name
+
+
+def _tail_inputs(S, H, D, seed):
+    g = torch.Generator().manual_seed(seed)
+    bf = lambda *s, std=1.0: (std * torch.randn(*s, generator=g)).to("cuda", torch.bfloat16)
+    dim = H * D
+    ang = 6.283 * torch.rand(S, D // 2, generator=g).cuda()
+    return dict(qx=bf(S, dim), kx=bf(S, dim), norm_q_w=1 + bf(dim, std=0.1),
+                norm_k_w=1 + bf(dim, std=0.1), cam=bf(S, 12), w_cam_q=bf(dim, 12, std=0.05),
+                w_cam_k=bf(dim, 12, std=0.05), cos=ang.cos(), sin=ang.sin(), dq=bf(S, H, D),
+                dk=bf(S, H, D))
+
+
+@pytest.mark.parametrize("frozen", ["both", "q", "k"])
+def test_prologue_backward_with_frozen_camera_weights(frozen):
+    """Camera weights that take no gradient change nothing in the others' (with
+    both frozen the pass keeps no camera sums)."""
+    need_gpu()
+    from multics_amd.kernels import qk_prologue_train
+    say("prologue backward, frozen camera weights", frozen)
+    S, H, D = 100, 4, 128
+    t = _tail_inputs(S, H, D, 5)
+    names = ["qx", "kx", "norm_q_w", "norm_k_w", "w_cam_q", "w_cam_k"]
+
+    def grads(off):
+        x = {n: t[n].clone().requires_grad_(n not in off) for n in names}
+        q, k = qk_prologue_train(x["qx"], x["kx"], norm_q_w=x["norm_q_w"], norm_k_w=x["norm_k_w"],
+                                 rope_cos=t["cos"], rope_sin=t["sin"], num_heads=H, eps=1e-6,
+                                 cam=t["cam"], w_cam_q=x["w_cam_q"], w_cam_k=x["w_cam_k"])
+        torch.autograd.backward([q, k], [t["dq"], t["dk"]])
+        return {n: x[n].grad for n in names}
+
+    off = {"both": {"w_cam_q", "w_cam_k"}, "q": {"w_cam_q"}, "k": {"w_cam_k"}}[frozen]
+    want, got = grads(set()), grads(off)
+    for n in names:
+        if n in off:
+            assert got[n] is None
+        else:
+            assert torch.equal(got[n], want[n]), n
+
+
+@pytest.mark.parametrize("S,H,D,tokens", [(1, 4, 128, 16), (37, 24, 128, 5), (1000, 8, 64, 16),
+                                          (130, 64, 64, 33)])
+def test_prologue_backward_partial_rows(S, H, D, tokens):
+    """``hier_qk_prologue_bwd``, whose caller adds the partial rows itself: the
+    projections' gradients are those of ``hier_qk_prologue_grads``, and the
+    rows' sums are its gain gradients before their rounding to bf16 (2^-8 of
+    the value, half a unit of 8 bits, and fp32 sums in another order)."""
+    need_gpu()
+    import ctypes as C
+
+    from multics_amd import _capi
+    say("prologue backward partial rows", S, H, D, tokens)
+    dim = H * D
+    t = _tail_inputs(S, H, D, 6)
+    new = lambda *s, dtype=torch.bfloat16: torch.full(s, float("nan"), dtype=dtype, device="cuda")
+    stream = _capi.stream_of(t["qx"].device)
+
+    def run(grads):
+        dqx, dkx = new(S, dim), new(S, dim)
+        a = _capi.HierPrologueBwdArgs(
+            S=S, H=H, D=D, eps=1e-6, C=12, tokens_per_wave=tokens, qx=t["qx"].data_ptr(),
+            kx=t["kx"].data_ptr(), cam=t["cam"].data_ptr(), w_cam_q=t["w_cam_q"].data_ptr(),
+            w_cam_k=t["w_cam_k"].data_ptr(), norm_q_w=t["norm_q_w"].data_ptr(),
+            norm_k_w=t["norm_k_w"].data_ptr(), rope_cos=t["cos"].data_ptr(),
+            rope_sin=t["sin"].data_ptr(), dq=t["dq"].data_ptr(), dk=t["dk"].data_ptr(), dq_ss=dim,
+            dq_sh=D, dk_ss=dim, dk_sh=D, dqx=dqx.data_ptr(), dkx=dkx.data_ptr())
+        rows = _capi.lib().hier_qk_prologue_bwd_waves(C.byref(a))
+        assert rows >= -(-S // tokens)
+        part = new(2, rows, dim, dtype=torch.float32)
+        a.dw_q_partial, a.dw_k_partial = part[0].data_ptr(), part[1].data_ptr()
+        dn = new(2, dim)
+        if grads:
+            g = _capi.HierPrologueGradArgs(dnorm_q=dn[0].data_ptr(), dnorm_k=dn[1].data_ptr())
+            _capi.call("hier_qk_prologue_grads", C.byref(a), C.byref(g), stream)
+        else:
+            _capi.call("hier_qk_prologue_bwd", C.byref(a), stream)
+        torch.cuda.synchronize()
+        return dqx, dkx, part.double().sum(1), dn.double()
+
+    dqx, dkx, sums, _ = run(False)
+    dqx2, dkx2, _, dn = run(True)
+    assert torch.equal(dqx, dqx2) and torch.equal(dkx, dkx2)
+    assert not dqx.isnan().any() and not sums.isnan().any()
+    assert ((dn - sums).abs() <= 2.0 ** -8 * sums.abs() + 1e-5 * sums.abs().max()).all()
