@@ -52,12 +52,16 @@ def test_frame_attention_edges(D, Lq):
     or all queries see, head counts that leave waves of a workgroup empty, and
     q / k / v as slices of larger tensors (heads before tokens for k),
     against float64.  Scores, weights and sums are fp32, so a result is off
-    by its own bf16 rounding (2^-9 of it) and fp32 terms far below 1e-3 of the
+    by its own bf16 rounding (2^-8 of it) and fp32 terms far below 1e-3 of the
     values' size."""
     need_gpu()
     g = torch.Generator().manual_seed(100 * D + Lq)
     n_block = 3
-    for B, H, Lk, W in ((3, 5, 1, -1), (2, 4, 24, 21), (1, 3, 31, 4), (2, 2, 33, 6), (1, 1, 64, -1),
+    # (a row group is 4 keys at D = 128, 8 at 64; a chunk 2, 3, 4, 6 or 8 of them)
+    for B, H, Lk, W in ((3, 5, 1, -1), (1, 3, 5, 30), (2, 1, 7, -1), (1, 2, 8, 12), (1, 3, 9, 30),
+                        (2, 2, 12, 21), (1, 1, 13, -1), (1, 3, 16, 30), (1, 2, 17, 12),
+                        (2, 4, 24, 21), (1, 3, 25, -1), (1, 3, 31, 4), (1, 1, 32, 30),
+                        (2, 2, 33, 6), (1, 2, 48, 21), (1, 1, 49, 12), (1, 1, 64, -1),
                         (2, 3, 65, 9), (1, 2, 200, 30)):
         say("frame attention edges", D, Lq, B, H, Lk, W)
         q = torch.randn(B, Lq + 2, H + 1, D, generator=g).to(torch.bfloat16)[:, 1:-1, 1:]
@@ -149,7 +153,7 @@ def test_frame_attention_weights_are_fp32(D, Lq):
     """Softmax weights multiply V with all their 24 bits in every kernel.  Keys
     of weight 1, p and 1 carry v = hi, -1 and lo, the bf16 of p and the bf16
     of what that leaves: the result is what two bf16 parts of p leave out,
-    over 2 + p.  Bound: the result's bf16 rounding (2^-9 of it) and the fp32
+    over 2 + p.  Bound: the result's bf16 rounding (2^-8 of it) and the fp32
     error of p (exp2 and score, 2^-23 together)."""
     need_gpu()
     say("frame attention weights", D, Lq)
@@ -168,7 +172,7 @@ def test_frame_attention_weights_are_fp32(D, Lq):
     ref = ((hi.double() - p + lo.double()) / (2 + p))[None, None, :, None].expand_as(got)
     assert (ref.abs() > 2.0 ** -21).sum() > ref.numel() / 4   # seen above the bound
     err = (got - ref).abs()
-    assert (err <= 2.0 ** -9 * ref.abs() + 2.0 ** -23).all(), float(err.max())
+    assert (err <= 2.0 ** -8 * ref.abs() + 2.0 ** -23).all(), float(err.max())
 
 
 @pytest.mark.parametrize("B,H,Lq", [(2_850_000, 24, 1), (16_800_000, 1, 17)])
