@@ -15,9 +15,19 @@ SLEEP = 20_000_000      # cycles: well above the time of a build
 
 
 def _arrays(t):
+    """What a launch reads: the items, the cut items and the lists that the
+    items address (entries between the lists are not written)."""
     n = t.n_items
-    return [x.cpu() for x in (t.items[:n], t.kv_idx, t.kv_mask, t.blk_and,
-                              M.launch_list(t).items[:n])]
+    items, cut, idx, msk, blk = (x.cpu() for x in (t.items[:n], M.launch_list(t).items[:n],
+                                                   t.kv_idx, t.kv_mask, t.blk_and))
+    return [items, cut] + [x for o, c in items[:, 5:7].tolist()
+                           for x in (idx[o:o + c], msk[o:o + c], blk[o // 64:(o + c) // 64])]
+
+
+def _same(got, want):
+    assert len(got) == len(want)
+    for i, (x, y) in enumerate(zip(got, want)):
+        assert torch.equal(x, y), i
 
 
 def _tiles():
@@ -50,7 +60,7 @@ def test_a_list_found_from_another_stream_is_complete(monkeypatch):
         hit = _tiles()
         assert hit is t
         got = _arrays(hit)                  # copies on b, waiting for b alone
-    assert all(torch.equal(x, y) for x, y in zip(got, want))
+    _same(got, want)
     # the key-major list, made by a's first backward, found by b's
     monkeypatch.setattr(_capi, "call", slow)
     with torch.cuda.stream(a):
@@ -60,7 +70,7 @@ def test_a_list_found_from_another_stream_is_complete(monkeypatch):
         assert M.backward_lists(t)[0] is kt
         got = _arrays(kt)
     torch.cuda.synchronize()
-    assert all(torch.equal(x, y) for x, y in zip(got, _arrays(kt)))
+    _same(got, _arrays(kt))
     assert int(kt.items[:, 6].sum()) > 0
 
 
@@ -72,18 +82,19 @@ def test_a_list_dropped_while_another_stream_reads_it():
     a, b = torch.cuda.Stream(), torch.cuda.Stream()
     with torch.cuda.stream(a):
         t = _tiles()
-    want = t.kv_idx.cpu()
+    torch.cuda.synchronize()
+    want = _arrays(t)[2]
     with torch.cuda.stream(b):
         hit = _tiles()
         torch.cuda._sleep(SLEEP)
         copy = hit.kv_idx.clone()
-    shape = t.kv_idx.shape
+    shape, (off, cnt) = t.kv_idx.shape, t.items[0, 5:7].tolist()
     M._LAYOUT_CACHE.clear()
     del t, hit
     with torch.cuda.stream(a):
         later = [torch.full(shape, -1, dtype=torch.int32, device="cuda") for _ in range(64)]
     torch.cuda.synchronize()
-    assert torch.equal(copy.cpu(), want) and len(later) == 64
+    assert torch.equal(copy.cpu()[off:off + cnt], want) and len(later) == 64
 
 
 def test_steps_of_one_plan_on_two_streams():
@@ -109,13 +120,9 @@ def test_steps_of_one_plan_on_two_streams():
             got.append(plan.build(lg))
     torch.cuda.synchronize()
 
-    def rows(t):                            # the lists proper: what the items address
-        items, idx, msk = t.items.cpu(), t.kv_idx.cpu(), t.kv_mask.cpu()
-        return [items] + [x[o:o + c] for o, c in items[:, 5:7].tolist() for x in (idx, msk)]
-
     for t, w in zip(got, want):
-        for x, y in ((t, w), (M.transpose_tiles(t), M.transpose_tiles(w))):
-            assert all(torch.equal(p, q) for p, q in zip(rows(x), rows(y)))
+        _same(_arrays(t), _arrays(w))
+        _same(_arrays(M.transpose_tiles(t)), _arrays(M.transpose_tiles(w)))
 
 
 def test_a_step_captured_in_a_graph_replays():
@@ -141,8 +148,5 @@ def test_a_step_captured_in_a_graph_replays():
         torch.cuda.synchronize()
         w = plan.build(logits)
         torch.cuda.synchronize()
-        for x, y in ((t, w), (M.transpose_tiles(t), M.transpose_tiles(w))):
-            assert torch.equal(x.items, y.items)
-            for o, c in x.items[:, 5:7].tolist():
-                assert torch.equal(x.kv_idx[o:o + c], y.kv_idx[o:o + c])
-                assert torch.equal(x.kv_mask[o:o + c], y.kv_mask[o:o + c])
+        _same(_arrays(t), _arrays(w))
+        _same(_arrays(M.transpose_tiles(t)), _arrays(M.transpose_tiles(w)))
