@@ -1660,6 +1660,8 @@ class MembershipLogitsPlan:
         self.ws_bytes = max(int(_capi.lib().hier_derive_workspace(C.byref(self._derive_args(sup)))), 1)
         self._steps: "OrderedDict[int, _StepBuffers]" = OrderedDict()   # by stream
         self._lock = threading.Lock()
+        if self.device.type == "cuda":              # the first step's, made with the plan
+            self._buffers(_capi.stream_of(self.device))
         self._ready = _ready.made(self)
 
     def kept_tensors(self):
