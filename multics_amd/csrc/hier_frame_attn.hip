@@ -20,14 +20,14 @@
 //               tokens per player): 128 queries per workgroup on the matrix
 //               cores, 64-key tiles of K and V in LDS, the next tile's rows
 //               loaded during the current one.  Bound by the latency of its
-//               few steps.  10 x 24 heads, 660 x 96 keys: 39 us (329 us with
+//               few steps.  10 x 24 heads, 660 x 96 keys: 40 us (329 us with
 //               one key at a time per query).
 //
 // Both give every key a weight, 0 where the mask hides it, and 0 times an
 // infinity or a NaN is a NaN.  A hidden row counts for nothing whatever it
 // holds, so where results are not all finite, or a query's weights sum to 0,
 // a wave computes its queries again from their visible keys alone, a key at a
-// time (visible_only).  The check costs the keyboard branch 2 us of 39, waves
+// time (visible_only).  The check costs the keyboard branch 2 us of 40, waves
 // of 7 or 8 queries 1-3 %, the temporal branch nothing.
 #include "hier_common.h"
 #include "hier_launch.h"

@@ -33,7 +33,7 @@
 // of its own dWc and adds the products there (slow, but no real camera changes
 // that often).  All sums are added in a fixed order.
 //
-// 18,816 tokens x 3,072 of q and k, camera on: 694 MB in 146 us (4.8 TB/s; a
+// 18,816 tokens x 3,072 of q and k, camera on: 694 MB in 146-150 us (4.6-4.8 TB/s; a
 // copy reaches 5.05) plus 9 us for the sums.  One wave per 16 tokens with no
 // loads ahead took 465 us, plus 26 us for the gain sums and 131 us for the
 // camera-weight gradients as two GEMMs over dx.
