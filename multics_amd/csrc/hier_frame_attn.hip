@@ -5,7 +5,8 @@
 // q_frame[i] - k_frame[j] < local_attn.  Scores, softmax weights and sums are
 // fp32 (the weights multiply V as three bf16 parts where the matrix cores do it).
 //
-// Two kernels, by the queries and keys of a sequence:
+// Three kernels, by the queries and keys of a sequence and by how many
+// sequences and heads there are:
 //
 // seq_kernel    few queries (the temporal branch: one sequence per spatial
 //               token, a block's 3 frames against a window of 24).  Bound by
@@ -16,6 +17,10 @@
 //               groups' sums at the end.  2,200 sequences x 24 heads of 128,
 //               3 x 24 keys: 115 us, 6.1 TB/s (155 us, 4.5 TB/s, when each
 //               query read the rows for itself, four keys at a time).
+// slot_kernel   a short window (a rollout's first blocks, small windows).  8 or
+//               4 queries per wave, each by D / 8 lanes, key after key.
+//               1,970 x 12 heads of 64, 3 x 8 keys: 17.5 us (23.2 as
+//               seq_kernel, whose fixed work is the larger part there).
 // tile_kernel   more (the keyboard branch: 660 video tokens against 96 keyboard
 //               tokens per player): 128 queries per workgroup on the matrix
 //               cores, 64-key tiles of K and V in LDS, the next tile's rows
@@ -23,7 +28,7 @@
 //               few steps.  10 x 24 heads, 660 x 96 keys: 40 us (329 us with
 //               one key at a time per query).
 //
-// Both give every key a weight, 0 where the mask hides it, and 0 times an
+// seq_kernel and tile_kernel give every key a weight, 0 where the mask hides it, and 0 times an
 // infinity or a NaN is a NaN.  A hidden row counts for nothing whatever it
 // holds, so where results are not all finite, or a query's weights sum to 0,
 // a wave computes its queries again from their visible keys alone, a key at a
@@ -131,6 +136,75 @@ __device__ __forceinline__ void visible_only(const HierFrameAttnArgs& a, int64_t
     if (mine)
       *reinterpret_cast<u32x4*>(a.o + b * a.o_sb + (int64_t)qi * a.o_ss + h * a.o_sh + 8 * c) = w;
   }
+}
+
+// ---- short windows -----------------------------------------------------------
+
+// A wave serves 64 / (D / 8) (sequence, query) slots of one head: D / 8 lanes
+// per query, each query over its own sequence's keys (slots of one sequence
+// read the same rows), four of them loaded before any is used.  Bound by its
+// instructions per query and key, and by one trip's latency per four keys; it
+// holds no rows and sums nothing across them, which on a short window is most of a seq_kernel wave's work.
+template <int D>
+__global__ __launch_bounds__(64) void slot_kernel(HierFrameAttnArgs a) {
+#pragma clang fp contract(off)   // (as in visible_only)
+  constexpr int LPR = D / 8, R = 64 / LPR, G = 4;
+  const int lane = threadIdx.x, c = lane % LPR, h = blockIdx.y;
+  const uint32_t slot = blockIdx.x * R + lane / LPR;      // (fewer than 2^28)
+  const bool mine = slot < (uint32_t)a.B * (uint32_t)a.Lq;
+  const uint32_t seq = mine ? slot / (uint32_t)a.Lq : 0u;
+  const int qi = mine ? (int)(slot - seq * (uint32_t)a.Lq) : 0;
+  const int64_t b = seq;
+  const u32x4 q = *reinterpret_cast<const u32x4*>(a.q + b * a.q_sb + (int64_t)qi * a.q_ss +
+                                                  (int64_t)h * a.q_sh + 8 * c);
+  Window win;
+  win.init(a.q_frame[qi], a.n_block, a.local_attn);
+  const uint16_t* const kb = a.k + b * a.k_sb + (int64_t)h * a.k_sh + 8 * c;
+  const uint16_t* const vb = a.v + b * a.v_sb + (int64_t)h * a.v_sh + 8 * c;
+  const float c2 = a.scale * kLog2e;
+  float m = -INFINITY, l = 0.f, o[8] = {};
+  for (int j0 = 0; j0 < a.Lk; j0 += G) {
+    u32x4 k[G], v[G];
+    int kf[G];
+#pragma unroll
+    for (int u = 0; u < G; ++u) {
+      const int j = min(j0 + u, a.Lk - 1);
+      k[u] = *reinterpret_cast<const u32x4*>(kb + (int64_t)j * a.k_ss);
+      v[u] = *reinterpret_cast<const u32x4*>(vb + (int64_t)j * a.v_ss);
+      kf[u] = a.k_frame[j];
+    }
+#pragma unroll
+    for (int u = 0; u < G; ++u) {
+      if (j0 + u >= a.Lk) break;
+      float s = 0.f;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const uint32_t x = q[e], y = k[u][e];
+        s = __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2, x),
+                                            __builtin_bit_cast(bf16x2, y), s, false);
+      }
+#pragma unroll
+      for (int d = 1; d < LPR; d <<= 1) s += __shfl_xor(s, d, 64);
+      if (!win.sees(kf[u])) continue;
+      const float t = s * c2, mn = fmaxf(m, t);
+      const float alpha = __builtin_amdgcn_exp2f(m - mn);   // m = -inf: 0
+      const float p = __builtin_amdgcn_exp2f(t - mn);
+      l = fmaf(l, alpha, p);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        o[2 * e] = fmaf(p, lo(v[u][e]), o[2 * e] * alpha);
+        o[2 * e + 1] = fmaf(p, hi(v[u][e]), o[2 * e + 1] * alpha);
+      }
+      m = mn;
+    }
+  }
+  if (!mine) return;
+  const float inv = l > 0.f ? 1.f / l : 0.f;
+  u32x4 w;
+#pragma unroll
+  for (int e = 0; e < 4; ++e)
+    w[e] = (uint32_t)f2bf(o[2 * e] * inv) | ((uint32_t)f2bf(o[2 * e + 1] * inv) << 16);
+  *reinterpret_cast<u32x4*>(a.o + b * a.o_sb + (int64_t)qi * a.o_ss + (int64_t)h * a.o_sh + 8 * c) = w;
 }
 
 // ---- up to 8 queries per sequence ------------------------------------------
@@ -475,6 +549,27 @@ __global__ __launch_bounds__(256, 2) void tile_kernel(HierFrameAttnArgs a, int q
 // 64 keys), 4 where it loops over chunks (each waits for its rows).
 bool one_chunk(const HierFrameAttnArgs& a) { return a.Lk <= 8 * (512 / a.D); }
 int query_groups(const HierFrameAttnArgs& a) { return one_chunk(a) ? (a.Lq + 7) / 8 : (a.Lq + 3) / 4; }
+// slot_kernel's time goes with queries x keys; a seq_kernel wave costs a chunk
+// of 16 keys (D = 64) or 8 (128) at least, a tile_kernel workgroup 32 x 32, and
+// with few sequences the chip waits for slot_kernel's trips of four keys.
+// slot_kernel / seq_kernel, us: D = 64, 23,640 (sequence, head) pairs: 1 query x
+// 1 key 4.9 / 13.8, 3 x 3 9.5 / 22.7, 3 x 8 17.5 / 23.2, 7 x 12 38 / 40, 3 x 15
+// 28.5 / 25.1; 4,800 pairs: 3 x 3 4.8 / 7.2, 3 x 8 7.1 / 7.3, 3 x 12 8.8 / 7.5, 16 x 12
+// 17.4 / 19.8; 1,600: 1 x 4 3.4 / 3.7, 3 x 8 5.8 / 4.7, 16 x 10 9.0 / 10.1; 800: 1 x 4
+// 3.4 / 3.1.  D = 128, 23,640: 3 x 3 18.2 / 22.5, 4 x 4 24.9 / 26.1, 3 x 6 27.7 /
+// 24.1; 3,600: 3 x 4 6.7 / 6.5, 8 x 4 8.7 / 10.4.
+// slot_kernel / tile_kernel, D = 128: 240 pairs: 660 x 3 27.7 / 30.9, 660 x 6
+// 38.3 / 31.2, 20 x 6 5.9 / 5.3; 1,600: 24 x 10 16.6 / 17.1, 48 x 5 18.5 / 22.4, 48 x
+// 8 22.5 / 22.3; 24,000: 17 x 12 150 / 217, 32 x 8 202 / 240, 32 x 10 246 / 241.
+bool use_slots(const HierFrameAttnArgs& a) {
+  const int64_t pairs = (int64_t)a.B * a.H;
+  if ((int64_t)a.B * a.Lq >= 1ll << 28) return false;   // its grid along x
+  if (a.Lq > 16) return a.Lk <= 4 || ((int64_t)a.Lq * a.Lk <= 256 && pairs >= 512);
+  if (a.Lk <= 2) return true;
+  const int64_t queries = pairs * a.Lq;
+  if (a.D == 128) return a.Lk <= 4 && queries >= 8192;
+  return a.Lk <= 12 && queries >= (a.Lk <= 4 ? 2048 : a.Lk <= 8 ? 8192 : 20480);
+}
 // tile_kernel works on 32 queries whether they are there or not.  Windows of one
 // chunk (2,200 x 24 heads, 24 keys, D = 128), seq_kernel / tile_kernel: 8
 // queries 173 / 445 us, 16 309 / 475, 24 472 / 508, 32 612 / 533; 40 x 24 heads:
@@ -546,6 +641,13 @@ extern "C" int hier_frame_attn(const HierFrameAttnArgs* args, void* stream) {
   const hier::Grid gr = hier::launch_grid(hier::xcd_grid(wgs), 256);
   HIER_REQUIRE(wgs <= hier::kMaxLaunchItems && gr.x != 0, HIER_EUNSUPPORTED, "too many queries");
   const hipStream_t st = (hipStream_t)stream;
+  if (use_slots(a)) {
+    const int64_t groups = ((int64_t)a.B * a.Lq + 512 / a.D - 1) / (512 / a.D);
+    const dim3 sg((unsigned)groups, a.H);
+    if (a.D == 128) hipLaunchKernelGGL(slot_kernel<128>, sg, dim3(64), 0, st, a);
+    else hipLaunchKernelGGL(slot_kernel<64>, sg, dim3(64), 0, st, a);
+    return hier::check_launch("slot_kernel");
+  }
   if (use_seq(a)) {
     if (a.D == 128) launch_seq_d<128>(a, st);
     else launch_seq_d<64>(a, st);

@@ -179,18 +179,61 @@ def test_frame_attention_weights_are_fp32(D, Lq):
 def test_frame_attention_many_sequences(B, H, Lq):
     """More sequences and heads than a grid holds along x (2^26 waves; 2^24
     matrix-tile workgroups): every one is computed.  Inputs are one sequence's,
-    expanded; one key, so the output is its V row."""
+    expanded; so are its 20 keys, so the output is their V row."""
     need_gpu()
     say("frame attention many sequences", B, H, Lq)
     D = 64
     g = torch.Generator().manual_seed(H)
-    q, k, v = (torch.randn(1, L, H, D, generator=g).to("cuda", torch.bfloat16).expand(B, L, H, D)
-               for L in (Lq, 1, 1))
-    got = frame_attention(q, k, v, torch.zeros(Lq), torch.zeros(1), 1, -1)
+    q, k, v = (torch.randn(1, n, H, D, generator=g).to("cuda", torch.bfloat16).expand(B, L, H, D)
+               for n, L in ((Lq, Lq), (1, 20), (1, 20)))
+    got = frame_attention(q, k, v, torch.zeros(Lq), torch.zeros(20), 1, -1)
     torch.cuda.synchronize()
     step = 9973
     for part in (got[::step], got[-2:], got[B // 2:B // 2 + 2]):
-        assert torch.equal(part, v[:1].expand_as(part))
+        assert torch.equal(part, v[:1, :1].expand_as(part))
+
+
+@pytest.mark.parametrize("B,H,Lq,Lk,D", [
+    # up to 16 queries: 2 keys; at D = 64 windows of up to 4, 8 and 12 keys from
+    # 2,048, 8,192 and 20,480 queries (of all sequences and heads) on; fewer
+    # queries or a key more: the other kernels
+    (1, 1, 1, 1, 128), (3, 5, 5, 2, 64), (2, 3, 9, 2, 128), (342, 6, 1, 4, 64), (341, 6, 1, 4, 64), (683, 6, 3, 4, 64), (683, 6, 2, 8, 64),
+    (682, 6, 2, 8, 64), (683, 6, 7, 5, 64), (683, 6, 2, 9, 64), (1707, 6, 2, 12, 64),
+    (1706, 6, 2, 12, 64), (1707, 6, 2, 13, 64), (214, 6, 16, 12, 64),
+    # at D = 128: 4 keys from 8,192 queries on
+    (683, 6, 2, 4, 128), (682, 6, 2, 4, 128), (683, 6, 3, 1, 128), (683, 6, 3, 5, 128),
+    # more queries: 4 keys, or queries x keys up to 256 with 512 pairs
+    (1, 3, 17, 1, 64), (2, 2, 660, 4, 128), (256, 2, 32, 8, 64), (256, 2, 51, 5, 128),
+    (256, 2, 17, 16, 128), (255, 2, 32, 8, 128)])
+def test_frame_attention_short_windows(B, H, Lq, Lk, D):
+    """The kernel of short windows and the edges of its range, with keys that
+    no query, one query or all queries see (a NaN in a row that none sees),
+    lanes past the last query and strided q / k / v, against float64.  Bounds
+    as in test_frame_attention_edges."""
+    need_gpu()
+    say("frame attention short windows", B, H, Lq, Lk, D)
+    g = torch.Generator("cuda").manual_seed(B + Lq + Lk + D)
+    rnd = lambda *s: torch.randn(*s, generator=g, device="cuda").to(torch.bfloat16)
+    q = rnd(B, Lq + 1, H + 1, D)[:, 1:, 1:]
+    k = rnd(B, H, Lk, D).transpose(1, 2)
+    v = rnd(B, Lk, 2 * H, D)[:, :, :H]
+    kf = (5 + 2 * torch.arange(Lk)) // 3
+    qf = 1 + torch.arange(Lq) * (int(kf[-1]) + 2) // Lq
+    m = kf[None] <= qf[:, None]
+    if Lk > 2:
+        m &= qf[:, None] - kf[None] < 4
+    dark = ~m.any(0)
+    kk, vv = k.clone(), v.clone()
+    kk[:, dark], vv[:, dark] = float("nan"), float("inf")
+    got = frame_attention(q, kk, vv, qf, kf, 1, 4 if Lk > 2 else -1).double()
+    torch.cuda.synchronize()
+    t = lambda x: x.double().transpose(1, 2).contiguous()
+    sc = t(q) @ t(k).transpose(2, 3).contiguous() / math.sqrt(D)
+    p = torch.softmax(sc.masked_fill(~m.cuda(), -math.inf), -1).nan_to_num(0.0)
+    ref = (p @ t(v)).transpose(1, 2)
+    err = (got - ref).abs()
+    assert (err <= 2.0 ** -8 * ref.abs() + 1e-3).all(), float(err.max())
+    assert (got[:, (~m.any(1)).cuda()] == 0).all()
 
 
 class _Attn(nn.Module):
