@@ -605,7 +605,7 @@ void launch_seq_d(const HierFrameAttnArgs& a, hipStream_t st) {
     case 2: return launch_seq<D, 2, true>(a, st);
     case 3: return launch_seq<D, 3, true>(a, st);
     case 4: return launch_seq<D, 4, true>(a, st);
-    case 5:
+    case 5: HIER_NQ(5);
     case 6: HIER_NQ(6);
     // (7 as 8, 1,970 x 12 heads, 14 keys, D = 64: 50.9 us, as 7 46.9)
     case 7: HIER_NQ(7);
