@@ -11,11 +11,14 @@
 //
 // One pass over HBM: x and y read once, out written once (out may be x).
 // Each thread moves 16-byte chunks (8 channels); the grid strides over the
-// rows x (dim / 8) chunks.  STREAM (the three tensors exceed the 256 MiB
-// last-level cache, so neither the producer's y nor this pass's out survives in
-// it whole): non-temporal loads and stores.  4 x 9,240 rows x 3,072 (681 MB)
-// 126 -> 118 us, 5.8 TB/s; 1.7 GB 333 -> 317 us; 341 MB 62.3 -> 60.2.  Smaller
-// ones stay in the cache: 195 MB 30.8 us plain, 35.3 streamed.
+// rows x (dim / 8) chunks.  STREAM (the distinct tensors exceed 320 MiB, a
+// quarter more than the last-level cache, of which a pass that follows then finds
+// nothing): non-temporal loads and stores.  4 x 9,240 rows x 3,072 (681 MB)
+// 126 -> 118 us, 5.8 TB/s.  Plain / streamed, the same buffers again and again:
+// 260 MB 42.4 / 47.0 us, 300 49.4 / 53.5, 340 62.7 / 60.2, 500 93 / 87; buffers in
+// turn: 300 52.6 / 54.6, 340 62.2 / 61.0, 500 94 / 87.  In place (two tensors),
+// again and again: 280 MB 70.5 / 77.9 us, 333 79.4 / 86.7, 400 106 / 104, 467 133
+// / 123; in turn: 280 84.6 / 77.3, 333 95.7 / 86.9, 400 115 / 105.
 #include "hier_common.h"
 
 #include <algorithm>
@@ -78,7 +81,8 @@ extern "C" int hier_gated_residual(const HierGateArgs* args, void* stream) {
   const int64_t n = a.rows * cpr;
   // about eight chunks per thread: enough loads in flight, few waves
   const int64_t blocks = std::min<int64_t>((n + 2047) / 2048, 256 * 32);
-  if (3 * 16 * n > (256ll << 20))
+  const int64_t tensors = a.out == a.x || a.out == a.y ? 2 : 3;
+  if (tensors * 16 * n > (320ll << 20))
     hipLaunchKernelGGL(gate_kernel<true>, dim3((unsigned)blocks), dim3(256), 0, (hipStream_t)stream,
                        a, n, cpr);
   else
