@@ -16,14 +16,29 @@ captures) and nothing made is kept: it holds nothing until the graph runs."""
 from __future__ import annotations
 
 import dataclasses
-import threading
 
 import torch
 
 from . import _capi
 
-# guards the order of the kept dictionaries (a lookup moves its entry to the end)
-LOCK = threading.Lock()
+
+def touch(cache, key) -> None:
+    """Moves a kept entry to the end of its ordered dictionary, unless another
+    thread has evicted it since it was found."""
+    try:
+        cache.move_to_end(key)
+    except KeyError:
+        pass
+
+
+def evict(cache, n: int) -> None:
+    """Drops the oldest entries until at most ``n`` are left (several threads
+    may, and then drop no more than one too many each)."""
+    while len(cache) > n:
+        try:
+            cache.popitem(last=False)
+        except KeyError:
+            return
 
 
 def capturing(device) -> bool:

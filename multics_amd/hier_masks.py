@@ -66,12 +66,10 @@ def _cache_put(key, value):
     n = int(os.environ.get("WAN_HIER_BLOCKMASK_CACHE_SIZE", "2"))
     if n == 0 or _ready.being_captured(value):
         return value
-    ready = _ready.made(value)
-    with _ready.LOCK:
-        _MASK_CACHE[key] = (value, ready)
-        _MASK_CACHE.move_to_end(key)
-        while 0 < n < len(_MASK_CACHE):
-            _MASK_CACHE.popitem(last=False)
+    _MASK_CACHE[key] = (value, _ready.made(value))
+    _ready.touch(_MASK_CACHE, key)
+    if n > 0:
+        _ready.evict(_MASK_CACHE, n)
     return value
 
 

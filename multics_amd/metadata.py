@@ -1438,13 +1438,12 @@ _LAYOUT_CACHE: "OrderedDict[tuple, object]" = OrderedDict()
 
 def _lru_get(cache, key):
     """The kept value, for use on the current stream."""
-    with _ready.LOCK:
-        hit = cache.get(key)
-        if hit is None:
-            return None
-        cache.move_to_end(key)
+    hit = cache.get(key)
+    if hit is None:
+        return None
+    _ready.touch(cache, key)
     value, ready = hit
-    if ready is not None:
+    if ready is not None and _capi.stream_of(ready.device) not in ready.streams:
         ready.join(value)
     return value
 
@@ -1454,12 +1453,9 @@ def _lru_put(cache, key, value, env, default):
     n = max(int(os.environ.get(env, default)), 0)
     if n == 0 or _ready.being_captured(value):
         return
-    ready = _ready.made(value)
-    with _ready.LOCK:
-        cache[key] = (value, ready)
-        cache.move_to_end(key)
-        while len(cache) > n:
-            cache.popitem(last=False)
+    cache[key] = (value, _ready.made(value))
+    _ready.touch(cache, key)
+    _ready.evict(cache, n)
 
 
 def _freeze(x):

@@ -135,18 +135,15 @@ def freqs_to_cos_sin(freqs: torch.Tensor, device=None):
     version counter, the device and the stream)."""
     dev = torch.device(device) if device is not None else freqs.device
     key = (id(freqs), freqs._version, str(dev), _capi.stream_of(dev) if dev.type == "cuda" else 0)
-    with _ready.LOCK:
-        hit = _COS_SIN_CACHE.get(key)
-        if hit is not None and hit[0] is freqs:
-            _COS_SIN_CACHE.move_to_end(key)
-            return hit[1], hit[2]
+    hit = _COS_SIN_CACHE.get(key)
+    if hit is not None and hit[0] is freqs:
+        _ready.touch(_COS_SIN_CACHE, key)
+        return hit[1], hit[2]
     f = freqs.reshape(freqs.shape[0], -1)
     if device is not None:
         f = f.to(device)
     cs, sn = f.real.to(torch.float32).contiguous(), f.imag.to(torch.float32).contiguous()
     if not freqs.requires_grad and not _ready.capturing(dev):
-        with _ready.LOCK:
-            _COS_SIN_CACHE[key] = (freqs, cs, sn)
-            while len(_COS_SIN_CACHE) > _COS_SIN_CACHE_SIZE:
-                _COS_SIN_CACHE.popitem(last=False)
+        _COS_SIN_CACHE[key] = (freqs, cs, sn)
+        _ready.evict(_COS_SIN_CACHE, _COS_SIN_CACHE_SIZE)
     return cs, sn

@@ -176,3 +176,33 @@ def test_steps_on_two_streams_write_their_own_buffers(gpu, monkeypatch):
     gpu.capturing = True                             # a graph's buffers are nobody else's
     t, g = step(1)
     assert all(g[f] != a[f] for f in a) and t._keepalive[1].ws.data_ptr() == g["ws"]
+
+
+def test_threads_share_a_small_cache(monkeypatch):
+    """Lookups move entries that other threads evict meanwhile."""
+    import sys
+    import threading
+    monkeypatch.setenv("WAN_HIER_SEGMENTED_META_CACHE_SIZE", "1")
+    cache, errors = type(M._META_CACHE)(), []
+
+    def work(i):
+        try:
+            for j in range(20000):
+                k = (i + j) % 3
+                v = M._lru_get(cache, k)
+                assert v is None or v == ("value", k)
+                M._lru_put(cache, k, ("value", k), "WAN_HIER_SEGMENTED_META_CACHE_SIZE", "64")
+        except BaseException as e:      # noqa: B036 (reported below)
+            errors.append(e)
+
+    old = sys.getswitchinterval()
+    sys.setswitchinterval(1e-6)
+    try:
+        threads = [threading.Thread(target=work, args=(i,)) for i in range(4)]
+        for t in threads:
+            t.start()
+        for t in threads:
+            t.join()
+    finally:
+        sys.setswitchinterval(old)
+    assert not errors and len(cache) <= 1
